@@ -390,6 +390,9 @@ class DotPipeline:
         plr_env = os.environ.get("NEWT_PLR", "auto")
         state["plr"] = S >= 3 and (plr_env == "1" or (plr_env == "auto" and simple))
         state["simple"] = simple
+        # the accumulator's name when the body is `acc = nl.dot(a, b, acc)`:
+        # waves left over by the output tile may then split k (staged_dot)
+        state["acc_name"] = self._dot_accumulator(compute[0]) if simple else None
         # a loop body with a dot and an exponential (flash attention) takes
         # LLVM's exp/MFMA interleave strategy in its branch-free copy
         state["exp_mix"] = ndots > 0 and any(_callee(nd) in ("exp", "exp2")
@@ -446,6 +449,8 @@ class DotPipeline:
             self.emit("newt::wait_vmcnt<0>();")
         if state["plr"]:
             self._insert_lines(mark, self._plr_preamble(state, n))
+        if state.get("ksplit"):
+            self._join_ksplit(state, mark)
         self._exit_compound(rec)
         self.end_loop_target(node)
         self.after_loop(node)
@@ -458,6 +463,63 @@ class DotPipeline:
         for r in self.pending_hoist:
             if r["index"] >= index:
                 r["index"] += len(lines)
+
+    @staticmethod
+    def _dot_accumulator(s):
+        """Name of the accumulator of a statement `acc = nl.dot(a, b, acc)`."""
+        if not (isinstance(s, ast.Assign) and _callee(s.value) == "dot"):
+            return None
+        c = s.value
+        acc = c.args[2] if len(c.args) == 3 else next(
+            (k.value for k in c.keywords if k.arg == "acc"), None)
+        name = _target(s)
+        return name if isinstance(acc, ast.Name) and acc.id == name else None
+
+    def _ksplit(self, state, acc, Lc, nks, rep):
+        """Whether the `rep` groups of waves that the output tile leaves over
+        split a k-step's MFMAs between them (nks of them per stage). Each
+        group then accumulates its share of k for the whole tile, and
+        _join_ksplit adds the shares after the loop. A loop whose carried
+        accumulator has not learned the MFMA layout yet computes the tile in
+        every group (this pass only teaches the layout)."""
+        if state.get("acc_name") is None or nks % rep:
+            self._no_pipe(state)
+        split = isinstance(acc, Reg) and acc.storage and acc.layout == Lc and bool(acc.vec)
+        if state.setdefault("ksplit", split and {"acc": acc, "rep": rep, "L": Lc}) \
+                and not split:
+            self._no_pipe(state)
+        return split and bool(state["ksplit"])
+
+    def _join_ksplit(self, state, mark):
+        """Around a loop whose waves split k: every group but the first starts
+        from zero, and afterwards each group adds all shares, in group order
+        (so every wave holds the same sums), through the stages' LDS.
+
+        This is for output tiles too small to give every wave rows or columns
+        of its own (16x16 to 64x64 per workgroup, a product with few rows):
+        such a launch is bound by how many bytes of the long operand are in
+        flight, which grows with the waves and the depth of the k-step, and
+        its MFMAs are few. x[16,4096] @ w[4096,4096].t() in bf16 took 58 us
+        on 64x64 tiles (64 workgroups, one 64-deep k-step in flight at a time
+        per barrier)."""
+        info = state["ksplit"]
+        acc, rep, L = info["acc"], info["rep"], info["L"]
+        nv, lanes = L.nslots // acc.vec, self.T // rep
+        group = f"(_tid / {lanes})"
+        zero = "f32x16" if acc.vec == 16 else "f32x4"
+        self._insert_lines(mark, [f"if ({group}) {{"]
+                           + [f"  {acc.var}[{i}] = ({zero})(0.0f);" for i in range(nv)] + ["}"])
+        nbytes = 4 * self.T * L.nslots
+        if nbytes <= state["stage_bytes"]:
+            area = state["names"][0]
+        else:
+            area = f"(_lds + {self.lds_arena(nbytes)})"
+        # every wave's copies have landed and every wave is done with the stages
+        self.emit("newt::wait_vmcnt<0>();")
+        self.emit("__syncthreads();")
+        self.emit(f"newt::join_k_groups<{acc.vec}, {nv}, {rep}, {lanes}>({acc.var}, "
+                  f"(f32x4*){area}, _tid);")
+        self.emit("__syncthreads();")
 
     def _plr_preamble(self, state, n):
         """Declarations of the prefetched fragments and their first fill from
@@ -797,7 +859,7 @@ class DotPipeline:
             idx.append(i)
         if reused or self.loop_depth > 0:
             self.emit("__syncthreads();")
-        state.update(recs=recs, ops=ops, names=names, lds_idx=idx)
+        state.update(recs=recs, ops=ops, names=names, lds_idx=idx, stage_bytes=off)
 
     def pipe_issue(self, state, slot, valid, fast=False):
         if state["recs"] is None:
@@ -956,12 +1018,16 @@ class DotPipeline:
         (lanes 32-63): a lane's four k of one row are contiguous, one 16-byte
         read of a K-major tile (four 4-byte reads of an R-major one) feeds four
         MFMAs, and both operands use the same order."""
-        if rep > 1 or instr != "32x32x2" or K % 8:
+        if instr != "32x32x2" or K % 8:
             self._no_pipe(state)
         Bt = Staged(b.rec, b.slot, not b.trans) if isinstance(b, Staged) else None
         if not isinstance(a, Staged) or Bt is None:
             self._no_pipe(state)
-        Lc = self.mfma_layout(M, N, instr, wm, wn, 1)
+        Lc = self.mfma_layout(M, N, instr, wm, wn, rep)
+        ng, k0 = K // 8, ""
+        if rep > 1 and self._ksplit(state, acc, Lc, ng, rep):
+            ng //= rep
+            k0 = f" + (_wave >> {lo.log2i(wm * wn)}) * {K // rep}"
         RM, RN = M // wm // 32, N // wn // 32
         orient = self.dot_orient()
         accv = self.init_acc(node, acc, Lc, M, N)
@@ -980,6 +1046,7 @@ class DotPipeline:
         def group(idx, X, r0, kk):
             # the record describes the tile's [R, K] view (R = M for A, N for B)
             rec, tile = X.rec, tiles[idx]
+            kk = f"{kk}{k0}"
             if rec["fmt"] == "k":
                 return f"newt::lds_frag_k32f<{rec['K']}>({tile}, {r0}, {kk}, _lane)"
             c = f"({r0} + (_lane & 31))"
@@ -987,7 +1054,7 @@ class DotPipeline:
                             for t in range(4))
             return f"f32x4{{{els}}}"
 
-        for g in range(K // 8):
+        for g in range(ng):
             kk = 8 * g
             for i in range(RM):
                 self.emit(f"const f32x4 _fa{g}_{i} = {group(0, a, f'_ra + {i * 32}', kk)};")
@@ -1084,15 +1151,21 @@ class DotPipeline:
         state = getattr(self, "pipe_active", None)
         if dt == tp.float32 and state is not None:
             return self._staged_dot_f32(node, a, b, acc, M, N, K, instr, wm, wn, rep, state)
-        if rep > 1 or kpl != 8 or dt not in (tp.float16, tp.bfloat16) or state is None:
+        if kpl != 8 or dt not in (tp.float16, tp.bfloat16) or state is None:
             if state is not None:
                 self._no_pipe(state)
             self.err(node, "internal: staged operand in an unsupported dot")
-        Lc = self.mfma_layout(M, N, instr, wm, wn, 1)
+        Lc = self.mfma_layout(M, N, instr, wm, wn, rep)
         T = dt.ctype
         Bt = Staged(b.rec, b.slot, not b.trans) if isinstance(b, Staged) else self.permute(b, (1, 0))
         RM, RN = M // wm // MI, N // wn // NI
-        nks = K // KI
+        nks, k0 = K // KI, ""
+        if rep > 1:
+            if not (isinstance(a, Staged) and isinstance(Bt, Staged)):
+                self._no_pipe(state)
+            if self._ksplit(state, acc, Lc, nks, rep):
+                nks //= rep
+                k0 = f" + (_wave >> {lo.log2i(wm * wn)}) * {K // rep}"
         orient = self.dot_orient()
         # an accumulator-layout A operand (fp16/bf16 cast of a row-per-lane dot
         # result) is used in place, with B read in the permuted k order: the
@@ -1144,7 +1217,7 @@ class DotPipeline:
                 else:
                     fn, targs = ((f"lds_frag_r_perm{MI}", f"{T}, {rec['R']}, {rec['sb']}") if perm
                                  else ("lds_frag_r", f"{T}, {rec['R']}, {MI}, {rec['sb']}"))
-                return f"newt::{fn}<{targs}>({tile}, {r0}, {kk}, _lane)"
+                return f"newt::{fn}<{targs}>({tile}, {r0}, {kk}{k0}, _lane)"
             if kind == "acc":
                 step = 8 if MI == 32 else 16
                 slots = [self._slot_for(X.layout, {0: i * MI, 1: kk + step * (e // 4) + (e % 4)})

@@ -422,7 +422,7 @@ __device__ __forceinline__ f32x4 mfma_16x16x4(float a, float b, f32x4 c) {
 // l / 32) puts two lanes of one cycle on one slot:
 //   64-byte rows:  q ^ ((q & 1) << 1), q = (r >> 2) & 3;
 //   128-byte rows: (r >> 1) & 7;
-//   256-byte rows: r & 15 (every key of fewer bits leaves a conflict: the
+//   256-byte rows and longer: r & 15 (every key of fewer bits leaves a conflict: the
 //   key's null space must avoid the lane offsets that share a cycle).
 // All three are conflict-free for both patterns.
 // ---------------------------------------------------------------------------
@@ -436,7 +436,7 @@ struct LdsTile {
   __host__ __device__ __forceinline__ static int key(int r) {
     const int q = (r >> SHIFT) & SWZ;
     if constexpr (CPR == 4) return q ^ ((q & 1) << 1);
-    else if constexpr (CPR == 16) return r & 15;
+    else if constexpr (CPR >= 16) return r & 15;
     else return q;
   }
   // element offset of (row r, reduction index k)
@@ -651,6 +651,34 @@ template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt range");
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
+
+// Sums of REP groups of LANES threads that each hold a share of the same
+// tile: thread t of every group holds NV vectors of V floats of the same
+// elements. Every group gets the sum of all shares, taken in group order, so
+// all groups hold the same bits. buf: REP * LANES * NV * V floats of LDS,
+// written with 16-byte accesses by consecutive lanes.
+template <int V, int NV, int REP, int LANES, typename VT>
+__device__ __forceinline__ void join_k_groups(VT* acc, f32x4* buf, int tid) {
+  const int g = tid / LANES, t = tid % LANES;
+  constexpr int Q = V / 4;
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+      buf[((i * Q + q) * REP + g) * LANES + t] =
+          f32x4{acc[i][4 * q], acc[i][4 * q + 1], acc[i][4 * q + 2], acc[i][4 * q + 3]};
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      f32x4 s = buf[(i * Q + q) * REP * LANES + t];
+#pragma unroll
+      for (int r = 1; r < REP; ++r) s += buf[((i * Q + q) * REP + r) * LANES + t];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[i][4 * q + e] = s[e];
+    }
 }
 
 // Workgroup barrier without the fence __syncthreads() carries. That fence

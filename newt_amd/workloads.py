@@ -192,10 +192,44 @@ MATMUL_CONFIGS = [
     newt.Config({"BLOCK_M": 64, "BLOCK_N": 128, "BLOCK_K": 64}, num_warps=4, num_stages=3),
     # 64x64 tiles give a 1024^3 problem 256 workgroups (one per CU)
     newt.Config({"BLOCK_M": 64, "BLOCK_N": 64, "BLOCK_K": 64}, num_warps=4, num_stages=4),
-    newt.Config({"BLOCK_M": 64, "BLOCK_N": 64, "BLOCK_K": 64}, num_warps=4, num_stages=3),
+    # 128-deep k-steps (128 KB of stages) halve the barriers: bf16 256x4096x4096
+    # 16.3 against 17.8 us for the tile above (x @ w.t(): 14.8 against 18.0),
+    # 1024x1024x4096 the same, 1024^3 7.0 either way
+    newt.Config({"BLOCK_M": 64, "BLOCK_N": 64, "BLOCK_K": 128}, num_warps=4, num_stages=4),
+    # two waves per SIMD over a 64x128 tile: bf16 640x2048x2048 (320 such
+    # tiles) 12.7 us against 15.1 for 64x64x64 and 15.5 for 128x128x64
+    newt.Config({"BLOCK_M": 64, "BLOCK_N": 128, "BLOCK_K": 64}, num_warps=8, num_stages=4),
 ]
 
 matmul_tuned = newt.autotune(configs=MATMUL_CONFIGS, key=["M", "N", "K"])(matmul_kernel)
+
+# Products whose 64x64 tiles do not fill the 256 CUs (few rows, few columns or
+# small all round) are bound by the bytes that the launch keeps in flight, not
+# by MFMAs: a 16-row product reads its long operand once. These tiles are
+# small enough for a workgroup per CU, their k-steps deep enough that each CU
+# keeps 50-100 KB of copies in flight, and waves that a tile has no rows or
+# columns for split k (DotPipeline._join_ksplit). bf16, back to back, against
+# the fastest of MATMUL_CONFIGS: x[16,4096] @ w[4096,4096].t() 7.9 against
+# 58 us (34 MB: 4.3 TB/s), 64 rows 9.3, 128 rows 12.5; w not transposed 12.1,
+# 12.2, 13.9; [32,8192] @ [8192,1024] 8.1 transposed, 18.3 not; 256x256x1024
+# 3.6 and 512x1024x1024 5.1 (5.6). 16-wide column tiles serve only a
+# transposed w (a tile of whole 16-byte runs along k); from 256 64x64 tiles on
+# (256x4096x4096, 1024^3) none of these wins.
+MATMUL_CONFIGS_SMALL = [
+    newt.Config({"BLOCK_M": 16, "BLOCK_N": 16, "BLOCK_K": 256}, num_warps=4, num_stages=4),
+    newt.Config({"BLOCK_M": 16, "BLOCK_N": 16, "BLOCK_K": 512}, num_warps=4, num_stages=4),
+    newt.Config({"BLOCK_M": 16, "BLOCK_N": 32, "BLOCK_K": 256}, num_warps=4, num_stages=4),
+    newt.Config({"BLOCK_M": 16, "BLOCK_N": 32, "BLOCK_K": 128}, num_warps=4, num_stages=6),
+    newt.Config({"BLOCK_M": 16, "BLOCK_N": 64, "BLOCK_K": 128}, num_warps=4, num_stages=4),
+    newt.Config({"BLOCK_M": 32, "BLOCK_N": 32, "BLOCK_K": 128}, num_warps=4, num_stages=4),
+    newt.Config({"BLOCK_M": 32, "BLOCK_N": 32, "BLOCK_K": 128}, num_warps=4, num_stages=6),
+    newt.Config({"BLOCK_M": 32, "BLOCK_N": 64, "BLOCK_K": 128}, num_warps=4, num_stages=4),
+    newt.Config({"BLOCK_M": 64, "BLOCK_N": 32, "BLOCK_K": 128}, num_warps=4, num_stages=4),
+    newt.Config({"BLOCK_M": 64, "BLOCK_N": 64, "BLOCK_K": 64}, num_warps=4, num_stages=4),
+    newt.Config({"BLOCK_M": 64, "BLOCK_N": 64, "BLOCK_K": 128}, num_warps=4, num_stages=4),
+]
+matmul_tuned_small = newt.autotune(configs=MATMUL_CONFIGS_SMALL,
+                                   key=["M", "N", "K"])(matmul_kernel)
 
 # fp32 operands run on the fp32 MFMA (v_mfma_f32_32x32x2_f32, full precision;
 # gfx950 has no tf32) through the same pipelined k-loop: 16-deep k-steps keep
@@ -218,7 +252,13 @@ def matmul(a, b, c=None, config=None):
             c.stride(0), c.stride(1))
     if config is None:
         grid = lambda meta: (newt.cdiv(M, meta["BLOCK_M"]), newt.cdiv(N, meta["BLOCK_N"]))
-        (matmul_tuned_fp32 if a.dtype == torch.float32 else matmul_tuned)[grid](*args)
+        if a.dtype == torch.float32:
+            tuned = matmul_tuned_fp32
+        elif newt.cdiv(M, 64) * newt.cdiv(N, 64) < 256:
+            tuned = matmul_tuned_small
+        else:
+            tuned = matmul_tuned
+        tuned[grid](*args)
     else:
         grid = (newt.cdiv(M, config.kwargs["BLOCK_M"]), newt.cdiv(N, config.kwargs["BLOCK_N"]))
         matmul_kernel[grid](*args, **config.kwargs, num_warps=config.num_warps,
