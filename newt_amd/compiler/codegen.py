@@ -454,6 +454,14 @@ class Codegen(ast.NodeVisitor):
             return ("and", [self._meta_expand(m, axis) for m in meta[1]])
         return None
 
+    def _meta_permute(self, meta, perm):
+        if meta[0] == "and":
+            parts = [self._meta_permute(m, perm) for m in meta[1]]
+            return None if any(m is None for m in parts) else ("and", parts)
+        if meta[0] == "cmp" and len(meta[2].shape) == len(perm):
+            return ("cmp", meta[1], self.permute(meta[2], perm))
+        return None
+
     def permute(self, v, perm):
         if isinstance(v, (Const, Scalar)):
             return v
@@ -478,7 +486,8 @@ class Codegen(ast.NodeVisitor):
             args = [self.permute(self.expand_to_rank(a, len(perm)), perm) if isinstance(a, Block) else a
                     for a in v.args]
             out = Lazy(v.dtype, shape, v.fn, args, v.size)
-            out.meta = None
+            meta = getattr(v, "meta", None)
+            out.meta = meta and self._meta_permute(meta, perm)
             return out
         if isinstance(v, PtrBlock):
             return PtrBlock(v.base, self.permute(v.offset, perm))

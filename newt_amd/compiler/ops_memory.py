@@ -128,8 +128,9 @@ class MemoryOps:
             div = min(div, min(c.div * cd, 1 << 30))
         return div
 
-    def mask_all_true(self, mask, shape):
-        """Uniform C condition under which `mask` is true everywhere, or None."""
+    def mask_all_true(self, mask, shape, parts=None):
+        """Uniform C condition under which `mask` is true everywhere, or None.
+        parts: only these of a conjunction's comparisons (indexes)."""
         if mask is None:
             return "true"
         if isinstance(mask, Const):
@@ -140,7 +141,9 @@ class MemoryOps:
         if not meta or meta[0] != "and":
             return None
         conds = []
-        for part in meta[1]:
+        for i, part in enumerate(meta[1]):
+            if parts is not None and i not in parts:
+                continue
             if part is None or part[0] != "cmp":
                 return None
             _, sym, aff = part
@@ -163,6 +166,42 @@ class MemoryOps:
             e = f"({base} + {ext})" if ext else f"({base})"
             conds.append(f"({e} {sym} 0)")
         return " && ".join(conds) if conds else "true"
+
+    def chunk_mask(self, mask, cdim, epc):
+        """The comparisons of `mask` when each has one value over every aligned
+        run of epc elements along dim cdim (meta parts, as mask_all_true reads
+        them), else None. A comparison that does not depend on cdim has; so
+        has `base + index < 0` (or >= 0) with a unit coefficient and a base
+        that is a multiple of epc: both sides of the bound start on a run."""
+        meta = getattr(mask, "meta", None) if isinstance(mask, Lazy) else None
+        if not meta or meta[0] != "and":
+            return None
+        for part in meta[1]:
+            if part is None or part[0] != "cmp" or part[1] not in ("<", "<=", ">", ">="):
+                return None
+            _, sym, aff = part
+            c = aff.coefs.get(cdim) if aff.shape[cdim] > 1 else None
+            if c is None:
+                continue
+            others = [v for a, v in aff.coefs.items() if a != cdim and aff.shape[a] > 1]
+            if not (c.is_const and c.const == 1 and sym in ("<", ">=") and aff.base.div % epc == 0
+                    and all(v.div % epc == 0 for v in others)):
+                return None
+        return meta[1]
+
+    @staticmethod
+    def mask_expr(parts, names):
+        """C condition of meta comparisons at the coordinates `names` (dim ->
+        C expression)."""
+        out = []
+        for _, sym, aff in parts:
+            terms = [aff.base.expr]
+            for a, c in sorted(aff.coefs.items()):
+                if aff.shape[a] > 1:
+                    terms.append(names[a] if c.is_const and c.const == 1
+                                 else f"{c.expr} * {names[a]}")
+            out.append(f"({' + '.join(terms)} {sym} 0)")
+        return " && ".join(out) or "true"
 
     # ------------------------------------------------------------ emission
     def emit_load(self, ld, L):

@@ -17,9 +17,17 @@ the K and V tiles of flash attention):
     of them before each LDS read;
   * a tile that is contiguous along one dim, 16-byte aligned and proven in
     bounds by a uniform test is copied global -> LDS with
-    global_load_lds_dwordx4 (no VGPR staging, no ds_write); other tiles
-    (ragged edges, strided operands) take a register path with the masked
-    loads' `other` fill, written with ds_write and hinted cold;
+    global_load_lds_dwordx4 (no VGPR staging, no ds_write); so is a ragged
+    tile whose mask is uniform over 16-byte chunks and fills with zero, its
+    masked chunks zeroed by an offset past the buffer descriptor's range (on
+    the register path, whose loads every iteration waited for, a ragged edge
+    ran 2-4x slower than a whole tile and the launch waited for it: fp16
+    1000x1024x776 14.5 -> 6.8 us on 64x64x64 tiles, 1319x1600x1280 32.5 ->
+    13.8, 777x1000x1032 26.6 -> 8.3, 4100x4104x4096 296 -> 157; causal
+    attention [4,32,4096,128], whose register tail spilled, 570 -> 555);
+    other tiles (strided operands, masks or bounds inside a chunk) take a
+    register path with the masked loads' `other` fill, written with ds_write
+    and hinted cold;
   * a tile is stored with its memory-contiguous dim contiguous in LDS: when
     that dim is the dot's reduction dim it is an XOR-swizzled K-major tile read
     with ds_read_b128, otherwise an R-major tile read with ds_read_b64_tr_b16
@@ -46,11 +54,12 @@ read after the loop (the advances run S-1 iterations ahead).
 """
 
 import ast
+import math
 import os
 
 from . import layouts as lo
 from . import types as tp
-from .values import Affine, Block, Const, LazyLoad, Reg, Scalar, Staged, Sym
+from .values import Affine, Block, Const, Fill, Lazy, LazyLoad, Reg, Scalar, Staged, Sym
 
 _SIDE_EFFECTS = {"store", "atomic_add", "atomic_max", "atomic_min"}
 
@@ -365,8 +374,30 @@ class DotPipeline:
                     changed = True
         return {"flat": flat, "staged": staged, "slice": sorted(slice_idx),
                 "advance": sorted(advance_idx), "konly": konly,
-                "kname": kname, "node": node, "fast_ok": fast_ok,
+                "kname": kname, "node": node, "fast_ok": fast_ok, "kinds": kinds,
                 "wheres": wheres, "where_deps": sorted(where_deps)}
+
+    def _mask_forms(self, e, plan):
+        """_kform of each comparison of a staged mask, in the order in which
+        the mask's value lists them (chunk_mask), or None when the expression
+        is not a conjunction of comparisons."""
+        kinds, flat = plan["kinds"], plan["flat"]
+        if isinstance(e, ast.BinOp) and isinstance(e.op, ast.BitAnd):
+            a, b = self._mask_forms(e.left, plan), self._mask_forms(e.right, plan)
+            return None if a is None or b is None else a + b
+        if isinstance(e, ast.Compare) and len(e.ops) == 1:
+            return [_kform(e, kinds)]
+        if isinstance(e, ast.Subscript):
+            return self._mask_forms(e.value, plan)
+        if isinstance(e, ast.Name):
+            if e.id in plan["konly"]:
+                s = next(s for s in flat if _target(s) == e.id)
+                return self._mask_forms(s.value, plan)
+            v = self.locals.get(e.id)
+            meta = getattr(v, "meta", None) if isinstance(v, Lazy) else None
+            if kinds.get(e.id, "c") == "c" and meta and meta[0] == "and":
+                return ["c"] * len(meta[1])
+        return None
 
     # ----------------------------------------------------------- emission
     def pipelined_for(self, node, plan, lo_, hi, st, idt):
@@ -662,7 +693,11 @@ class DotPipeline:
             if not isinstance(X, LazyLoad) or X.result is not None or tuple(X.shape) != r["shape"]:
                 self._no_pipe(state)
             if r["dma"]:
-                full = self.mask_all_true(X.mask, X.shape)
+                # comparisons that no iteration changes are left to the copies
+                parts = None
+                if r["inv"] and state.get("bufdma"):
+                    parts = set(range(len(X.mask.meta[1]))) - set(r["inv"])
+                full = self.mask_all_true(X.mask, X.shape, parts)
                 if full is not None and full != "true":
                     conds.append(f"({full})")
                 if full is not None and state.get("bufdma"):
@@ -792,6 +827,26 @@ class DotPipeline:
             return False
         return (R * K // epc) % self.T == 0
 
+    def _dma_mask(self, X, V, fmt, dt, info, plan):
+        """(whether a direct-to-LDS tile can be copied under its mask, the
+        mask's comparisons that no iteration changes). The copy drops a masked
+        16-byte chunk by an offset past the buffer's end, which writes zeros,
+        so the mask must be uniform over chunks and `other` zero."""
+        other = X.other
+        if isinstance(other, Fill):
+            other = other.value
+        if not (other is None or (isinstance(other, Const) and other.pyval == 0)):
+            return False, ()
+        parts = self.chunk_mask(V.mask, 1 if fmt == "k" else 0, 16 // dt.itemsize)
+        if parts is None or os.environ.get("NEWT_BUFFER_DMA", "1") == "0":
+            return False, ()
+        call = plan["flat"][info["index"]].value
+        masks = [k.value for k in call.keywords if k.arg == "mask"] + list(call.args[1:2])
+        forms = self._mask_forms(masks[0], plan) if masks else None
+        if forms is None or len(forms) != len(parts):
+            return True, ()
+        return True, tuple(i for i, f in enumerate(forms) if f == "c")
+
     def _r_tile_swizzle_bit(self, info, fmt, R, K, dt):
         """Swizzle bit of a 16-bit R-major tile: 2 when its dot will most
         likely read it with the accumulator-ordered 16-row fragments (a B
@@ -831,7 +886,9 @@ class DotPipeline:
             epc = 16 // dt.itemsize
             if dma:
                 ops += R * K // epc // self.T
+            masked, inv = self._dma_mask(X, V, fmt, dt, info, state["plan"]) if dma else (False, ())
             recs[nm] = {"name": nm, "shape": tuple(X.shape), "dt": dt, "kdim": kdim, "R": R,
+                        "masked": masked, "inv": inv,
                         "K": K, "fmt": fmt, "off": off, "dma": dma,
                         "sb": self._r_tile_swizzle_bit(info, fmt, R, K, dt)}
             off += (nbytes + 15) // 16 * 16
@@ -839,6 +896,14 @@ class DotPipeline:
                 V.consumed = True
                 if V in self.pending_loads:
                     self.pending_loads.remove(V)
+        # A copy under a mask keeps a lane offset of its own in a VGPR for the
+        # whole loop. Wave tiles with 128 accumulator registers and more have
+        # none to spare (256x256x32 on 4 waves: 3 spilled registers -> 28), so
+        # their ragged programs run the general loop and the branch-free one
+        # stays for whole tiles; smaller tiles copy under the mask in both.
+        if len(recs) != 2 or math.prod(r["R"] for r in recs.values()) > 64 * self.T:
+            for r in recs.values():
+                r["inv"] = ()
         # stage arrays of a pipelined loop that has finished are reused (a
         # later loop never needs them at the same time); a barrier first lets
         # every wave finish reading them before this loop's copies land. A loop
@@ -879,8 +944,33 @@ class DotPipeline:
             tile = f"(({dt.ctype}*)({base} + {r['off']}))"
             full = self.mask_all_true(X.mask, X.shape) if r["dma"] else None
             if r["dma"] and full is not None and fast:
-                self._dma_stage(V, base, r["off"], fmt, R, K, dt, buffer=state.get("bufdma", False),
-                                sb=r["sb"])
+                buf = state.get("bufdma", False)
+                pred = None
+                if buf and r["inv"] and full != "true":
+                    pred = self.mask_expr([V.mask.meta[1][i] for i in r["inv"]], ("_r", "_k"))
+                self._dma_stage(V, base, r["off"], fmt, R, K, dt, buffer=buf, sb=r["sb"], pred=pred)
+            elif r["masked"] and full is not None and not fast:
+                # every chunk is copied or zero-filled by an asynchronous copy,
+                # so a ragged tile keeps the pipeline (and its wait counts)
+                pred = self.mask_expr(V.mask.meta[1], ("_r", "_k"))
+                self.emit(f"if (__builtin_expect({valid} && ({full}), 1)) {{")
+                self.indent += 1
+                self._dma_stage(V, base, r["off"], fmt, R, K, dt, sb=r["sb"])
+                self.indent -= 1
+                self.emit(f"}} else if ({valid}) {{")
+                self.indent += 1
+                self.emit(f"if (__builtin_expect({self._lane_bytes_fit(V, R, K, dt)}, 1)) {{")
+                self.indent += 1
+                self._dma_stage(V, base, r["off"], fmt, R, K, dt, buffer=True, sb=r["sb"], pred=pred)
+                self.indent -= 1
+                self.emit("} else {")
+                self.indent += 1
+                self._dma_stage(V, base, r["off"], fmt, R, K, dt, sb=r["sb"], pred=pred)
+                self.emit("newt::wait_vmcnt<0>();")
+                self.indent -= 1
+                self.emit("}")
+                self.indent -= 1
+                self.emit("}")
             elif fast:
                 self._reg_stage(V, tile, fmt, R, K, dt, sb=r["sb"])
             elif r["dma"] and full is not None:
@@ -930,10 +1020,13 @@ class DotPipeline:
         conds.append(f"({' + '.join(parts) if parts else '0LL'}) < {(1 << 31) // dt.itemsize}LL")
         return " && ".join(conds)
 
-    def _dma_stage(self, X, base, boff, fmt, R, K, dt, buffer=False, sb=3):
-        """Direct-to-LDS copies of one [R, K] tile. buffer: the branch-free
-        fast loop's form, a scalar descriptor on the tile's uniform start and
-        a 32-bit lane offset (the entry test guarantees it fits)."""
+    def _dma_stage(self, X, base, boff, fmt, R, K, dt, buffer=False, sb=3, pred=None):
+        """Direct-to-LDS copies of one [R, K] tile. buffer: a scalar descriptor
+        on the tile's uniform start and a 32-bit lane offset (the caller's test
+        guarantees it fits). pred: C condition of the 16-byte chunk at (_r, _k);
+        chunks where it is false become zeros, in the buffer form by an offset
+        past the descriptor's range, otherwise by a guarded load and an LDS
+        write (the caller drains that one)."""
         off = X.ptr.offset
         T = dt.ctype
         epc = 16 // dt.itemsize
@@ -961,11 +1054,18 @@ class DotPipeline:
             if buffer:
                 tb = f"({gb} + ({ubase}))" if ubase else gb
                 lb = f"(unsigned)(({' + '.join(lane) if lane else '0'}) * {dt.itemsize})"
-                self.emit(f"newt::lds_dma16_buf({tb}, {lb}, {dst});")
+                if pred:
+                    self.emit(f"newt::lds_dma16_masked({tb}, {lb}, {pred}, {dst});")
+                else:
+                    self.emit(f"newt::lds_dma16_buf({tb}, {lb}, {dst});")
             else:
                 terms = ([ubase] if ubase else []) + lane
                 gaddr = f"({gb} + {' + '.join(terms) if terms else '0'})"
-                self.emit(f"newt::lds_dma16({gaddr}, {dst});")
+                if pred:
+                    self.emit(f"newt::lds_copy16_if({gaddr}, {pred}, "
+                              f"(void*)({base} + {boff} + 16 * _s));")
+                else:
+                    self.emit(f"newt::lds_dma16({gaddr}, {dst});")
             self.indent -= 1
             self.emit("}")
 

@@ -645,6 +645,26 @@ __device__ __forceinline__ void lds_dma16_buf(const void* base, unsigned lane_by
                                            lane_bytes, 0, 0, 0);
 }
 
+// The same copy where `in` holds; elsewhere the lane's 16 bytes of LDS become
+// zeros: an offset of 2^31 lies past this descriptor's range (num_records
+// 2^31), and a buffer load out of range returns zeros without touching memory.
+// Callers keep lane_bytes + 16 within 2^31.
+__device__ __forceinline__ void lds_dma16_masked(const void* base, unsigned lane_bytes, bool in,
+                                                 void* wave_dst) {
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<void*>(base), (short)0, (int)0x80000000, 0x00020000);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)wave_dst, 16,
+                                           in ? lane_bytes : 0x80000000u, 0, 0, 0);
+}
+
+// lds_dma16_masked for lane offsets of any size, through a register: dst is
+// the lane's own 16 bytes.
+__device__ __forceinline__ void lds_copy16_if(const void* g, bool in, void* dst) {
+  u32x4 v = {0, 0, 0, 0};
+  if (in) v = *(const u32x4*)g;
+  *(u32x4*)dst = v;
+}
+
 // Wait until at most N vector-memory operations of this wave are outstanding
 // (s_waitcnt vmcnt(N); expcnt and lgkmcnt left unconstrained).
 template <int N>
