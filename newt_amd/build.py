@@ -62,6 +62,8 @@ extern "C" __global__ void __launch_bounds__(256) newt_header_check(
   const int l = threadIdx.x & 63;
   float v[4];
   newt::load_vec<float, 4>(f + 4 * l, v);
+  f16 u[8];
+  newt::load_vec<f16, 8>(a + l, u, newt::any_align());
   float s = v[0] + v[1] + v[2] + v[3];
   s = newt::lane_reduce<newt::Sum, 63>(s);
   float m = newt::lane_reduce<newt::Max, 63>(v[0]);
@@ -87,7 +89,8 @@ extern "C" __global__ void __launch_bounds__(256) newt_header_check(
   newt::store_vec<float, 4>(o + 4 * threadIdx.x, r);
   newt::atomic_max(o, s);
   newt::atomic_add(o + 1, m);
-  if (n > 0 && newt::aligned(o, 16)) o[2] = newt::to_f32(newt::to_bf16(s));
+  newt::store_vec<f16, 8>(reinterpret_cast<f16*>(o) + 1, u, newt::any_align());
+  if (n > 0) o[2] = newt::to_f32(newt::to_bf16(s));
 }
 """
 

@@ -13,8 +13,11 @@ and whether a run's first address is 16-byte aligned; those runs become single
 global_load_dwordx4 / global_store_dwordx4 transactions. Masks built from
 comparisons of affine indices with scalars are reduced to one uniform
 "whole tile in bounds" condition that selects an unmasked fast path; other
-tiles take a per-run path (vector access when the run is fully valid,
-predicated element accesses otherwise).
+tiles take a per-run path: one vector access under the run's mask where the
+mask is proven uniform over runs, else a vector access when the run is fully
+valid and predicated element accesses for the run that the bound cuts. A run
+whose 16-byte alignment is not proven (rows of an odd stride) is accessed
+with the same vector instructions at its element's alignment.
 """
 
 import os
@@ -189,6 +192,31 @@ class MemoryOps:
                 return None
         return meta[1]
 
+    def run_mask(self, mask, L, chunk):
+        """How `mask` runs over the aligned runs of `chunk` slots along the
+        contiguous dim of L: 'uniform' (one value per run), 'prefix' (true up
+        to some element, then false), 'interval' (true between two elements),
+        or None when that is not known."""
+        d = L.reg[0][0]
+        if self.chunk_mask(mask, d, chunk) is not None:
+            return "uniform"
+        meta = getattr(mask, "meta", None) if isinstance(mask, Lazy) else None
+        if not meta or meta[0] != "and":
+            return None
+        kind = "prefix"
+        for part in meta[1]:
+            if part is None or part[0] != "cmp" or part[1] not in ("<", "<=", ">", ">="):
+                return None
+            _, sym, aff = part
+            c = aff.coefs.get(d) if aff.shape[d] > 1 else None
+            if c is None:
+                continue
+            if not c.is_const:
+                return None
+            if (c.const > 0) != (sym in ("<", "<=")):
+                kind = "interval"
+        return kind
+
     @staticmethod
     def mask_expr(parts, names):
         """C condition of meta comparisons at the coordinates `names` (dim ->
@@ -202,6 +230,15 @@ class MemoryOps:
                                  else f"{c.expr} * {names[a]}")
             out.append(f"({' + '.join(terms)} {sym} 0)")
         return " && ".join(out) or "true"
+
+    def _mask_bools(self, mask, L, g, chunk, run):
+        """Emit _m0.. of a run of slots; the condition that all hold (its ends
+        decide for an interval of true elements)."""
+        for i in range(chunk):
+            self.emit(f"const bool _m{i} = {self.ev(mask, L, g + i)};")
+        if run is None:
+            return " && ".join(f"_m{i}" for i in range(chunk))
+        return f"_m{chunk - 1}" if run == "prefix" else f"_m0 && _m{chunk - 1}"
 
     # ------------------------------------------------------------ emission
     def emit_load(self, ld, L):
@@ -221,6 +258,8 @@ class MemoryOps:
         proven = ptr.base.aligned16 and div % chunk == 0
         all_true = self.mask_all_true(mask, L.shape)
         nt = id(ld.node) in getattr(self, "stream_loads", ())
+        run = self.run_mask(mask, L, chunk) if chunk > 1 else None
+        align = "" if proven else ", newt::any_align()"
         rd = (lambda e: f"__builtin_nontemporal_load(&{e})") if nt else (lambda e: e)
 
         def oth(s):
@@ -235,29 +274,29 @@ class MemoryOps:
                     addr = f"({base} + {o})"
                     self.emit("{")
                     self.indent += 1
-                    if masked:
-                        ms = [f"({self.ev(mask, L, g + i)})" for i in range(chunk)]
-                        for i, m in enumerate(ms):
-                            self.emit(f"const bool _m{i} = {m};")
-                        cond = " && ".join(f"_m{i}" for i in range(chunk))
-                    else:
-                        cond = ""
-                    if not proven:
-                        al = f"newt::aligned({addr}, {chunk * esz})"
-                        cond = f"{cond} && {al}" if cond else al
                     vec = (f"newt::load_vec{'_nt' if nt else ''}<{elem.ctype}, {chunk}>({addr}, "
-                           f"{out.var} + {g});")
-                    if not cond:
+                           f"{out.var} + {g}{align});")
+                    if not masked:
                         self.emit(vec)
+                    elif run == "uniform":
+                        self.emit(f"if ({self.ev(mask, L, g)}) {{ {vec} }} else {{")
+                        for i in range(chunk):
+                            self.emit(f"  {out.at(g + i)} = {oth(g + i)};")
+                        self.emit("}")
                     else:
+                        cond = self._mask_bools(mask, L, g, chunk, run)
                         self.emit(f"if ({cond}) {{ {vec} }} else {{")
                         self.indent += 1
+                        if run == "prefix":
+                            # past the first element a run holds only `other`
+                            for i in range(chunk):
+                                self.emit(f"{out.at(g + i)} = {oth(g + i)};")
+                            self.emit("if (_m0) {")
                         for i in range(chunk):
                             e = rd(f"{base}[{o} + {i}]")
-                            if masked:
-                                self.emit(f"{out.at(g + i)} = _m{i} ? {e} : {oth(g + i)};")
-                            else:
-                                self.emit(f"{out.at(g + i)} = {e};")
+                            self.emit(f"{out.at(g + i)} = _m{i} ? {e} : {oth(g + i)};")
+                        if run == "prefix":
+                            self.emit("}")
                         self.indent -= 1
                         self.emit("}")
                     self.indent -= 1
@@ -359,6 +398,7 @@ class MemoryOps:
         proven = pbase.aligned16 and div % chunk == 0
         all_true = self.mask_all_true(mask, L.shape)
         vd = self.cdtype(value)
+        mrun = self.run_mask(mask, L, chunk) if chunk > 1 else None
         # a matmul's C tile (a column-oriented dot accumulator: the kernel has
         # no row reductions) is stored once, by every workgroup at about the
         # same time, after its k-loop: the non-temporal hint keeps that burst
@@ -390,24 +430,23 @@ class MemoryOps:
                     self.emit(f"{elem.ctype} _w[{chunk}];")
                     for i in range(chunk):
                         self.emit(f"_w[{i}] = {val(g + i)};")
-                    conds = []
-                    if masked:
-                        for i in range(chunk):
-                            self.emit(f"const bool _m{i} = {self.ev(mask, L, g + i)};")
-                        conds.append(" && ".join(f"_m{i}" for i in range(chunk)))
-                    if not proven:
-                        conds.append(f"newt::aligned({addr}, {chunk * esz})")
-                    vec = f"newt::store_vec{'_nt' if nt else ''}<{elem.ctype}, {chunk}>({addr}, _w);"
-                    if conds:
-                        self.emit(f"if ({' && '.join(conds)}) {{ {vec} }} else {{")
+                    align = "" if proven else ", newt::any_align()"
+                    vec = (f"newt::store_vec{'_nt' if nt else ''}<{elem.ctype}, {chunk}>"
+                           f"({addr}, _w{align});")
+                    if not masked:
+                        self.emit(vec)
+                    elif mrun == "uniform":
+                        self.emit(f"if ({self.ev(mask, L, g)}) {{ {vec} }}")
+                    else:
+                        cond = self._mask_bools(mask, L, g, chunk, mrun)
+                        some = "if (_m0) " if mrun == "prefix" else ""
+                        self.emit(f"if ({cond}) {{ {vec} }} else {some}{{")
                         self.indent += 1
                         for i in range(chunk):
                             st = scalar_store(f"{o} + {i}", f"_w[{i}]")
-                            self.emit(f"if (_m{i}) {st}" if masked else st)
+                            self.emit(f"if (_m{i}) {st}")
                         self.indent -= 1
                         self.emit("}")
-                    else:
-                        self.emit(vec)
                     self.indent -= 1
                     self.emit("}")
                 else:

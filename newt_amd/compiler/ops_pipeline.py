@@ -429,6 +429,7 @@ class DotPipeline:
         state["exp_mix"] = ndots > 0 and any(_callee(nd) in ("exp", "exp2")
                                              for x in compute for nd in ast.walk(x))
         state["pf"] = {}
+        state["late"] = []
         self.pipe_records.append(state)
         for s in range(S - 1):
             self.locals[kname] = self.new_scalar(idt, f"({lo_e} + {s * stv})")
@@ -541,9 +542,8 @@ class DotPipeline:
         self._insert_lines(mark, [f"if ({group}) {{"]
                            + [f"  {acc.var}[{i}] = ({zero})(0.0f);" for i in range(nv)] + ["}"])
         nbytes = 4 * self.T * L.nslots
-        if nbytes <= state["stage_bytes"]:
-            area = state["names"][0]
-        else:
+        area, size = self.lds_arrays[state["lds_idx"][0]]
+        if nbytes > size:
             area = f"(_lds + {self.lds_arena(nbytes)})"
         # every wave's copies have landed and every wave is done with the stages
         self.emit("newt::wait_vmcnt<0>();")
@@ -779,6 +779,8 @@ class DotPipeline:
                 self.locals.pop(t, None)
             if plr:
                 self._plr_fill(state, (s + 1) % S)
+            if fast:
+                self._write_late(state)
             if fast and state["simple"] and os.environ.get("NEWT_SCHED", "1") != "0":
                 self._sched_hints(state)
         self.pipe_active = None
@@ -860,7 +862,6 @@ class DotPipeline:
 
     def _init_recs(self, state):
         recs = {}
-        off = 0
         ops = 0
         for nm, info in sorted(state["plan"]["staged"].items(), key=lambda kv: kv[1]["index"]):
             X = self.locals.get(nm)
@@ -881,7 +882,6 @@ class DotPipeline:
                 state["plr"] = False
                 if fmt == "r" and R % 64:
                     self._no_pipe(state)
-            nbytes = self.tile_bytes(R, K, dt)
             dma = self._dma_ok(V, fmt, R, K, dt) and os.environ.get("NEWT_LDS_DMA", "1") != "0"
             epc = 16 // dt.itemsize
             if dma:
@@ -889,9 +889,9 @@ class DotPipeline:
             masked, inv = self._dma_mask(X, V, fmt, dt, info, state["plan"]) if dma else (False, ())
             recs[nm] = {"name": nm, "shape": tuple(X.shape), "dt": dt, "kdim": kdim, "R": R,
                         "masked": masked, "inv": inv,
-                        "K": K, "fmt": fmt, "off": off, "dma": dma,
+                        "K": K, "fmt": fmt, "dma": dma,
+                        "bytes": (self.tile_bytes(R, K, dt) + 15) // 16 * 16,
                         "sb": self._r_tile_swizzle_bit(info, fmt, R, K, dt)}
-            off += (nbytes + 15) // 16 * 16
             if V is not X:
                 V.consumed = True
                 if V in self.pending_loads:
@@ -908,23 +908,27 @@ class DotPipeline:
         # later loop never needs them at the same time); a barrier first lets
         # every wave finish reading them before this loop's copies land. A loop
         # nested in another rewrites its stages on each outer trip: same barrier
+        size, at = sum(r["bytes"] for r in recs.values()), 0
+        for r in recs.values():
+            r["off"] = at
+            at += r["bytes"]
         names, idx = [], []
         reused = False
         for _ in range(state["S"]):
             if self.lds_pool:
                 i = self.lds_pool.pop(0)
                 nm, sz = self.lds_arrays[i]
-                self.lds_arrays[i] = (nm, max(sz, off))
+                self.lds_arrays[i] = (nm, max(sz, size))
                 reused = True
             else:
                 i = len(self.lds_arrays)
                 nm = f"_ldsP{i}"
-                self.lds_arrays.append((nm, off))
+                self.lds_arrays.append((nm, size))
             names.append(nm)
             idx.append(i)
         if reused or self.loop_depth > 0:
             self.emit("__syncthreads();")
-        state.update(recs=recs, ops=ops, names=names, lds_idx=idx, stage_bytes=off)
+        state.update(recs=recs, ops=ops, names=names, lds_idx=idx)
 
     def pipe_issue(self, state, slot, valid, fast=False):
         if state["recs"] is None:
@@ -972,7 +976,13 @@ class DotPipeline:
                 self.indent -= 1
                 self.emit("}")
             elif fast:
-                self._reg_stage(V, tile, fmt, R, K, dt, sb=r["sb"])
+                # loaded here, written to LDS after this iteration's MFMAs
+                # (_write_late): the loads' latency hides behind them
+                self.indent -= 1
+                self.emit("}")
+                state["late"].append((self._reg_load(V, fmt, R, dt), tile, dt, fmt, r["sb"]))
+                self.emit("{")
+                self.indent += 1
             elif r["dma"] and full is not None:
                 cond = valid if full == "true" else f"{valid} && ({full})"
                 # the in-bounds copy is the hot path; the hint moves the masked
@@ -1069,16 +1079,33 @@ class DotPipeline:
             self.indent -= 1
             self.emit("}")
 
-    def _reg_stage(self, X, tile, fmt, R, K, dt, sb=3):
+    def _reg_load(self, X, fmt, R, dt):
+        """A tile on the register path, loaded in the layout it is written to
+        LDS from."""
         if fmt == "k":
             L = self.staging_layout(X)
         else:
             v = 16 // dt.itemsize
-            L = lo.blocked((K, R), self.W, min(v, R)).permute((1, 0))
+            L = lo.blocked((X.shape[1], R), self.W, min(v, R)).permute((1, 0))
         r = self.emit_load(X, L)
-        if r.dtype != dt:
-            r = self.to_reg(r, r.layout, dt)
-        self.write_tile_to(r, tile, dt, fmt, sb)
+        return r if r.dtype == dt else self.to_reg(r, r.layout, dt)
+
+    def _reg_stage(self, X, tile, fmt, R, K, dt, sb=3):
+        self.write_tile_to(self._reg_load(X, fmt, R, dt), tile, dt, fmt, sb)
+
+    def _write_late(self, state):
+        """Write the register-path tiles that the branch-free loop loaded
+        before its MFMAs into their stage: no wave reads that stage again
+        before the next iteration's barrier, which also publishes it. Bound by
+        the load latency that one iteration's MFMAs do not cover. With 16-byte
+        loads at any alignment, fp16 1000x1003x777 (odd strides) takes 13.7 us
+        against 25.2 for the same tile with 2-byte loads waited for at once,
+        2048x2047x2049 72 against 149; aligned 1024x1024x768 takes 5.9."""
+        late, state["late"] = state["late"], []
+        if late:
+            self.emit("__builtin_amdgcn_sched_barrier(0);")
+        for r, tile, dt, fmt, sb in late:
+            self.write_tile_to(r, tile, dt, fmt, sb)
 
     def write_tile_to(self, r, tile, dt, fmt, sb=3):
         """Write register block r ([R, K] view) into an LDS tile of format fmt

@@ -115,8 +115,52 @@ __device__ __forceinline__ void store_vec_nt(T* __restrict__ p, const T* in) {
   __builtin_nontemporal_store(__builtin_bit_cast(R, v), reinterpret_cast<R*>(p));
 }
 
-__device__ __forceinline__ bool aligned(const void* p, int bytes) {
-  return (reinterpret_cast<u64>(p) & (u64)(bytes - 1)) == 0;
+// The same accesses where only the element's own alignment is known (rows of an
+// odd stride): global memory takes a 16-byte access at any element address,
+// and one that straddles two lines costs far less than the eight 2-byte (four
+// 4-byte) accesses it replaces.
+struct any_align {};
+
+template <typename T, int N> struct any_vec {
+  typedef typename raw_vec<sizeof(T) * N>::type R;
+  typedef R type __attribute__((aligned(sizeof(T))));
+};
+
+template <typename T, int N>
+__device__ __forceinline__ void load_vec(const T* __restrict__ p, T* out, any_align) {
+  typedef typename any_vec<T, N>::R R;
+  R r = *reinterpret_cast<const typename any_vec<T, N>::type*>(p);
+  vec_t<T, N> v = __builtin_bit_cast(vec_t<T, N>, r);
+#pragma unroll
+  for (int i = 0; i < N; ++i) out[i] = v.d[i];
+}
+
+template <typename T, int N>
+__device__ __forceinline__ void load_vec_nt(const T* __restrict__ p, T* out, any_align) {
+  typedef typename any_vec<T, N>::R R;
+  R r = __builtin_nontemporal_load(reinterpret_cast<const typename any_vec<T, N>::type*>(p));
+  vec_t<T, N> v = __builtin_bit_cast(vec_t<T, N>, r);
+#pragma unroll
+  for (int i = 0; i < N; ++i) out[i] = v.d[i];
+}
+
+template <typename T, int N>
+__device__ __forceinline__ void store_vec(T* __restrict__ p, const T* in, any_align) {
+  typedef typename any_vec<T, N>::R R;
+  vec_t<T, N> v;
+#pragma unroll
+  for (int i = 0; i < N; ++i) v.d[i] = in[i];
+  *reinterpret_cast<typename any_vec<T, N>::type*>(p) = __builtin_bit_cast(R, v);
+}
+
+template <typename T, int N>
+__device__ __forceinline__ void store_vec_nt(T* __restrict__ p, const T* in, any_align) {
+  typedef typename any_vec<T, N>::R R;
+  vec_t<T, N> v;
+#pragma unroll
+  for (int i = 0; i < N; ++i) v.d[i] = in[i];
+  __builtin_nontemporal_store(__builtin_bit_cast(R, v),
+                              reinterpret_cast<typename any_vec<T, N>::type*>(p));
 }
 
 // ---------------------------------------------------------------------------

@@ -83,3 +83,15 @@ def test_masked_rows_near_two_gib(lda, M):
 
 def test_fp32_masked_copies():
     case(50, 60, 100, 104, 64, 64, 64, 16, 4, 4, dtype=torch.float32)
+
+
+@pytest.mark.parametrize("tile", [(64, 64, 64, 8, 2), (64, 64, 64, 4, 4), (128, 128, 32, 4, 3),
+                                  (32, 64, 128, 4, 2)])
+@pytest.mark.parametrize("lda,ldb", [(1033, 64), (1040, 65), (1033, 67)])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (13, 9, 65), (31, 63, 1032), (64, 64, 1024)])
+def test_odd_strides(tile, lda, ldb, M, N, K):
+    """Rows of an odd stride: tiles loaded into registers at their elements'
+    alignment ahead of the MFMAs and written to LDS after them, beside tiles
+    that are copied asynchronously."""
+    BM, BN, BK, waves, stages = tile
+    case(min(M, BM), min(N, BN), K, lda, ldb, BM, BN, BK, waves, stages)
