@@ -244,8 +244,29 @@ MATMUL_CONFIGS_FP32 = [
     newt.Config({"BLOCK_M": 256, "BLOCK_N": 128, "BLOCK_K": 16}, num_warps=8, num_stages=4),
     newt.Config({"BLOCK_M": 128, "BLOCK_N": 128, "BLOCK_K": 32}, num_warps=4, num_stages=3),
     newt.Config({"BLOCK_M": 128, "BLOCK_N": 128, "BLOCK_K": 16}, num_warps=4, num_stages=4),
+    # two waves per SIMD: 2048^3 118.4 against 119.9 us for the tile above
+    newt.Config({"BLOCK_M": 128, "BLOCK_N": 128, "BLOCK_K": 32}, num_warps=8, num_stages=3),
 ]
 matmul_tuned_fp32 = newt.autotune(configs=MATMUL_CONFIGS_FP32, key=["M", "N", "K"])(matmul_kernel)
+
+# fp32 products whose 128x128 tiles do not fill the 256 CUs: the fp32 MFMA is
+# slow enough (64 cycles for 32x32x2) that a launch takes as long as its
+# busiest CU has MFMAs, so the tile is what divides the work most evenly.
+# 1024^3 (64 tiles of 128x128) 61.6 -> 21.3 us on 64x64x32, of 13.7 us of MFMA
+# work per CU; 512^3 7.1, x @ w.t() 5.5; [16,4096] @ [4096,4096] 33.1, x @ w.t()
+# 18.9 (67 MB; 32x32 tiles serve a transposed w only); 1500x700x1003 38.9.
+# From 256 tiles of 128x128 on (2048^3) the larger list is level or ahead.
+MATMUL_CONFIGS_FP32_SMALL = [
+    newt.Config({"BLOCK_M": 32, "BLOCK_N": 32, "BLOCK_K": 64}, num_warps=4, num_stages=4),
+    newt.Config({"BLOCK_M": 32, "BLOCK_N": 64, "BLOCK_K": 32}, num_warps=4, num_stages=4),
+    newt.Config({"BLOCK_M": 32, "BLOCK_N": 64, "BLOCK_K": 64}, num_warps=8, num_stages=4),
+    newt.Config({"BLOCK_M": 64, "BLOCK_N": 64, "BLOCK_K": 32}, num_warps=4, num_stages=4),
+    newt.Config({"BLOCK_M": 64, "BLOCK_N": 64, "BLOCK_K": 32}, num_warps=8, num_stages=4),
+    newt.Config({"BLOCK_M": 64, "BLOCK_N": 128, "BLOCK_K": 32}, num_warps=8, num_stages=4),
+    newt.Config({"BLOCK_M": 128, "BLOCK_N": 128, "BLOCK_K": 32}, num_warps=8, num_stages=3),
+]
+matmul_tuned_fp32_small = newt.autotune(configs=MATMUL_CONFIGS_FP32_SMALL,
+                                        key=["M", "N", "K"])(matmul_kernel)
 
 
 def matmul(a, b, c=None, config=None):
@@ -258,7 +279,8 @@ def matmul(a, b, c=None, config=None):
     if config is None:
         grid = lambda meta: (newt.cdiv(M, meta["BLOCK_M"]), newt.cdiv(N, meta["BLOCK_N"]))
         if a.dtype == torch.float32:
-            tuned = matmul_tuned_fp32
+            few = newt.cdiv(M, 128) * newt.cdiv(N, 128) < 256
+            tuned = matmul_tuned_fp32_small if few else matmul_tuned_fp32
         elif newt.cdiv(M, 64) * newt.cdiv(N, 64) < 256:
             tuned = matmul_tuned_small
         else:

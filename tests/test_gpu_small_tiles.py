@@ -65,6 +65,14 @@ def test_few_tiles_are_tuned_over_small_tiles(M, N, K, dtype):
     assert any(key[:3] == (M, N, K) for key in W.matmul_tuned_small.timings)
 
 
+@pytest.mark.parametrize("M,N,K", [(16, 512, 512), (1, 64, 96), (300, 129, 77), (1000, 1024, 40)])
+@pytest.mark.parametrize("tb", [True, False])
+def test_few_fp32_tiles_are_tuned_over_small_tiles(M, N, K, tb):
+    from newt_amd import workloads as W
+    check(M, N, K, False, tb, torch.float32, None)
+    assert any(key[:3] == (M, N, K) for key in W.matmul_tuned_fp32_small.timings)
+
+
 @newt.jit
 def init_and_two_loops_k(a_ptr, b_ptr, o_ptr, K, FULL, REST, INIT: nl.constexpr,
                          BM: nl.constexpr, BN: nl.constexpr, BK: nl.constexpr):
