@@ -484,6 +484,40 @@ def attention_plain_kernel(q_ptr, k_ptr, v_ptr, o_ptr, S, H, scale,
     nl.store(o_base + offs_m[:, None] * som + offs_d[None, :], acc, mask=qmask)
 
 
+def attention_tile(S, heads, D, causal):
+    """(query rows, waves) of a program of the default kernel at 64-key blocks.
+
+    256 rows on 8 waves share each K and V block between the most rows, but a
+    launch needs programs for 256 CUs. Smaller tiles of 16 rows per wave keep
+    4 or 8 waves on a CU's four SIMDs; they read K and V from LDS more often
+    per row, which costs a launch that fills the chip anyway 15-24% at head
+    dim 128 and 3-7% at 64 (where 128 rows on 4 waves run 1-2% ahead of 256).
+    Not causal: the tile with the least rows on the busiest CU, weighed by
+    those rates: bf16 [1,16,1000,128] 32.0 us on 256 rows, 22.4 on 128, 18.5
+    on 64; [1,8,4096,128] 100.9 / 75.2 / 85.9; [2,32,4096,128] 444 / 540 / 583;
+    fp16 [2,16,1000,64] 23.9 / 17.2 / 17.9; bf16 [3,8,1500,64] 32.6 / 32.3 /
+    28.9. Causal: programs differ in length (the last query block attends to
+    every key), so a tile also wants several programs per CU:
+    [2,32,2048,128] 76.7 / 89.8 / 91.8 (512 programs of 256 rows),
+    [1,32,2048,128] 57.9 / 45.6 / 50.3 (256), [1,8,4096,128] 97.4 / 66.5 /
+    59.3; [4,32,2048,64] 110.7 / 105.9 / 104.6, [2,16,2048,64] 42.6 / 32.4 /
+    30.7."""
+    wide = D > 64
+    programs = {rows: newt.cdiv(S, rows) * heads for rows in (256, 128, 64)}
+    waves = {256: 8, 128: 8 if wide else 4, 64: 4}
+    if causal:
+        if wide and programs[256] >= 512:
+            rows = 256
+        elif programs[128] >= (512 if wide else 1024):
+            rows = 128
+        else:
+            rows = 64
+    else:
+        rate = {256: 1.0, 128: 0.85, 64: 0.78} if wide else {256: 1.0, 128: 1.02, 64: 0.93}
+        rows = min(rate, key=lambda r: newt.cdiv(programs[r], 256) * r / rate[r])
+    return rows, waves[rows]
+
+
 def attention(q, k, v, causal=False, scale=None, out=None, BLOCK_M=None, BLOCK_N=64,
               num_warps=None, num_stages=2, waves_per_eu=2, plain=False):
     """Flash attention forward over [B, H, S, D] tensors (unit stride along D).
@@ -496,22 +530,26 @@ def attention(q, k, v, causal=False, scale=None, out=None, BLOCK_M=None, BLOCK_N
     Default tiles: 32 query rows per wave, two waves per SIMD, 256-row
     programs on 8 waves (one workgroup per CU shares each K and V block
     between all 8 waves); causal too, where two 128-row workgroups per CU
-    measured 2-3% slower (their register budget spills around the
-    online-softmax pass)."""
+    measured 2-3% slower. A launch of the default kernel too small for that
+    takes attention_tile's."""
+    B, H, S, D = q.shape
+    scale = D ** -0.5 if scale is None else float(scale)
+    plain = plain or not scale > 0
+    if (BLOCK_M is None and num_warps is None and not plain
+            and (BLOCK_N, num_stages, waves_per_eu) == (64, 2, 2)):
+        BLOCK_M, num_warps = attention_tile(S, B * H, D, causal)
     if BLOCK_M is None:
         BLOCK_M = 256
     if num_warps is None:
         num_warps = BLOCK_M // 32
-    B, H, S, D = q.shape
     for t in (q, k, v):
         if t.stride(3) != 1:
             raise ValueError("attention: q, k and v need unit stride along head_dim")
     out = torch.empty_like(q) if out is None else out
     if out.stride(3) != 1:
         raise ValueError("attention: out needs unit stride along head_dim")
-    scale = D ** -0.5 if scale is None else float(scale)
     grid = (newt.cdiv(S, BLOCK_M), B * H)
-    if plain or not scale > 0:
+    if plain:
         attention_plain_kernel[grid](q, k, v, out, S, H, scale,
                                      q.stride(0), q.stride(1), q.stride(2),
                                      k.stride(0), k.stride(1), k.stride(2),
