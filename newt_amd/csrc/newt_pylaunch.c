@@ -26,7 +26,8 @@
  * The key holds the same facts as the Python signature: positional
  * constexprs and every keyword argument (constexprs and launch options) by
  * type and value, per runtime argument its kind and the facts the code
- * generator specializes on, the current device and the codegen switches.
+ * generator specializes on, the current device and the codegen switches (as
+ * one int per combination of their values).
  */
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
@@ -44,6 +45,9 @@ static PyObject* g_getstream = NULL;  /* torch._C._cuda_getCurrentRawStream */
 static PyObject* g_environ = NULL;    /* os.environ._data */
 static PyObject* g_envkeys = NULL;    /* tuple of bytes: the codegen switches */
 static PyObject* g_tensor = NULL;     /* torch.Tensor */
+static PyObject* g_envs = NULL;       /* dict: switch values (tuple) -> small int */
+static PyObject* g_env_id = NULL;     /* the current values' int */
+static uint64_t g_env_version = 0;    /* version of os.environ._data it was read at */
 static PyObject* s_data_ptr = NULL;
 static PyObject* s_get_device = NULL;
 static PyObject* s_dtype = NULL;
@@ -83,6 +87,8 @@ static PyObject* py_init(PyObject* self, PyObject* args) {
   Py_XSETREF(g_environ, Py_NewRef(environ));
   Py_XSETREF(g_envkeys, Py_NewRef(envkeys));
   Py_XSETREF(g_tensor, Py_NewRef(tensor));
+  Py_CLEAR(g_env_id);
+  if (!g_envs && !(g_envs = PyDict_New())) return NULL;
   Py_RETURN_NONE;
 }
 
@@ -127,6 +133,43 @@ typedef struct {
   int32_t device;
   uint64_t dtype;
 } Rec;
+
+/* The codegen switches' current values as a small int that stands for them in
+   the key (one per combination seen). Reading the 24 switches and hashing
+   their tuple was a third of a launch's key, so they are read again only when
+   the dict behind os.environ has changed: every write to a dict gives it a
+   version no dict had before. Returns a borrowed reference. */
+static PyObject* env_id(void) {
+#if PY_VERSION_HEX < 0x030C0000
+  const uint64_t version = ((PyDictObject*)g_environ)->ma_version_tag;
+  if (g_env_id && version == g_env_version) return g_env_id;
+#endif
+  Py_ssize_t ne = PyTuple_GET_SIZE(g_envkeys);
+  PyObject* env = PyTuple_New(ne);
+  if (!env) return NULL;
+  for (Py_ssize_t i = 0; i < ne; i++) {
+    PyObject* val = PyDict_GetItemWithError(g_environ, PyTuple_GET_ITEM(g_envkeys, i));
+    if (!val && PyErr_Occurred()) {
+      Py_DECREF(env);
+      return NULL;
+    }
+    PyTuple_SET_ITEM(env, i, Py_NewRef(val ? val : Py_None));
+  }
+  PyObject* id = PyDict_GetItemWithError(g_envs, env); /* borrowed */
+  if (!id && !PyErr_Occurred()) {
+    PyObject* fresh = PyLong_FromSsize_t(PyDict_GET_SIZE(g_envs));
+    if (fresh && PyDict_SetItem(g_envs, env, fresh) == 0) id = PyDict_GetItemWithError(g_envs, env);
+    Py_XDECREF(fresh);
+  }
+  Py_DECREF(env);
+  if (!id) return NULL;
+  Py_INCREF(id);
+  Py_XSETREF(g_env_id, id);
+#if PY_VERSION_HEX < 0x030C0000
+  g_env_version = version;
+#endif
+  return g_env_id;
+}
 
 static PyObject* call_noargs(PyObject* obj, PyObject* name) {
   return PyObject_VectorcallMethod(name, &obj, 1 | PY_VECTORCALL_ARGUMENTS_OFFSET, NULL);
@@ -243,23 +286,13 @@ static PyObject* py_run(PyObject* self, PyObject* const* a, Py_ssize_t na) {
     }
   }
   {
-    Py_ssize_t ne = PyTuple_GET_SIZE(g_envkeys);
-    PyObject* env = PyTuple_New(ne);
+    PyObject* env = env_id();
     if (!env) goto done;
-    for (Py_ssize_t i = 0; i < ne; i++) {
-      PyObject* val = PyDict_GetItemWithError(g_environ, PyTuple_GET_ITEM(g_envkeys, i));
-      if (!val && PyErr_Occurred()) {
-        Py_DECREF(env);
-        goto done;
-      }
-      PyTuple_SET_ITEM(env, i, Py_NewRef(val ? val : Py_None));
-    }
     PyObject* bytes = PyBytes_FromStringAndSize((const char*)rec, sizeof(Rec) * (nargs + 1));
     PyObject* ex = bytes ? PyList_AsTuple(extra) : NULL;
     key = (bytes && ex) ? PyTuple_Pack(3, bytes, env, ex) : NULL;
     Py_XDECREF(bytes);
     Py_XDECREF(ex);
-    Py_DECREF(env);
     if (!key) goto done;
   }
   {

@@ -94,6 +94,25 @@ class _Specialization:
         self.traced = tracer.generate(kernel.fn, kernel.fndef, args)
         self.jit, self.digest = _load_source(kernel.__name__, self.traced)
         self.index = {name: i for i, name in enumerate(kernel.param_names)}
+        # the launch's arguments and the extents that its grid and spans read,
+        # each as one generated expression over the call's arguments
+        flat, extent = [], {}
+        for (entry, value) in ((e, args[self.index[e[1]]]) for e in self.traced.args):
+            i = self.index[entry[1]]
+            flat.append(f"a[{i}]")
+            if entry[0] == "tensor":
+                flat += [f"a[{i}].size({d})" for d in range(value.dim())]
+                flat += [f"a[{i}].stride({d})" for d in range(value.dim())]
+                extent.update((f"{entry[1]}_d{d}", f"a[{i}].size({d})")
+                              for d in range(value.dim()))
+            else:
+                extent[entry[1]] = f"a[{i}]"
+        self._flat = eval(f"lambda a: ({', '.join(flat)},)")
+
+        def read(symbol):
+            return f"int({extent[symbol]})" if symbol in extent else str(int(symbol))
+        self._grid = eval("lambda a, c: ({},)".format(", ".join(
+            f"-(-{read(d.extent)} // c[{d.const!r}])" for d in self.traced.grid)))
 
     def extents(self, args):
         out = {}
@@ -110,16 +129,6 @@ class _Specialization:
     def resolve(extents, symbol):
         return int(extents[symbol]) if symbol in extents else int(symbol)
 
-    def flat_args(self, args):
-        out = []
-        for entry in self.traced.args:
-            value = args[self.index[entry[1]]]
-            out.append(value)
-            if entry[0] == "tensor":
-                out.extend(int(s) for s in value.shape)
-                out.extend(int(s) for s in value.stride())
-        return out
-
     def span_sizes(self, extents):
         """Constexprs of whole-dimension tiles; the dimensions one tile spans
         must agree (x[t, :] * w[:] needs x.shape[1] == w.shape[0])."""
@@ -133,13 +142,11 @@ class _Specialization:
         return out
 
     def launch(self, args, cfg):
-        extents = self.extents(args)
         consts = {name: cfg[name] for name in self.traced.tunable}
-        consts.update(self.span_sizes(extents))
-        grid = tuple(-(-self.resolve(extents, d.extent) // consts[d.const])
-                     for d in self.traced.grid)
-        self.jit[grid](*self.flat_args(args), **consts, num_warps=cfg.num_warps,
-                       num_stages=cfg.num_stages)
+        if self.traced.spans:
+            consts.update(self.span_sizes(self.extents(args)))
+        self.jit[self._grid(args, consts)](*self._flat(args), **consts, num_warps=cfg.num_warps,
+                                           num_stages=cfg.num_stages)
 
 
 # ------------------------------------------------------------------ search space
@@ -401,6 +408,7 @@ class Kernel:
         self.trials = []        # the latest tuning's (Config, ms or None, note)
         self._specs = {}        # argument signature -> _Specialization
         self._chosen = {}       # tuning key -> Config
+        self._keys = {}         # (specialisation, shapes) -> tuning key
         self._last = None
 
     # ---- public API
@@ -430,8 +438,8 @@ class Kernel:
         return self.fn(*[EagerTensor(a) if torch.is_tensor(a) else a for a in args])
 
     def _specialize(self, args):
-        sig = tuple((a.dim(), str(a.dtype)) if torch.is_tensor(a) else type(a).__name__
-                    for a in args)
+        sig = tuple([(a.dim(), a.dtype) if isinstance(a, torch.Tensor) else type(a).__name__
+                     for a in args])
         spec = self._specs.get(sig)
         if spec is None:
             spec = self._specs[sig] = _Specialization(self, args)
@@ -453,7 +461,10 @@ class Kernel:
         return SearchSpace(spec.traced, footprint)
 
     def _choose(self, spec, args):
-        key = self.tuning_key(spec, args)
+        quick = (spec, tuple([a.shape for a in args if isinstance(a, torch.Tensor)]))
+        key = self._keys.get(quick)
+        if key is None:
+            key = self._keys[quick] = self.tuning_key(spec, args)
         cfg = self._chosen.get(key)
         if cfg is None:
             cfg = _STORE.get(key)

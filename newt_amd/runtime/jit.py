@@ -422,6 +422,17 @@ class JITFunction:
                       consts)
         return ck, values
 
+    def _grid_of(self, grid, args, kwargs):
+        """A callable grid's value for this call (META: the arguments and
+        constexprs by name, defaults included, and num_warps)."""
+        meta = dict(self.defaults)
+        meta.update(zip(self.param_names, args))
+        meta.update(kwargs)
+        meta.setdefault("num_warps", 4)
+        meta.pop("num_stages", None)
+        meta.pop("waves_per_eu", None)
+        return grid(meta)
+
     def _run(self, grid, *args, **kwargs):
         ckey = None
         C = _C_LAUNCH if _C_LAUNCH is not None else _c_launcher()
@@ -431,6 +442,8 @@ class JITFunction:
             except (RuntimeError, AssertionError):
                 pass                # no GPU: the Python path reports what is wrong
         if C and _Dev.ready and launch_events is None:
+            if callable(grid):
+                grid = self._grid_of(grid, args, kwargs)
             try:
                 r = C.run(self._ctable, self._cx_pos, grid, args, kwargs)
             except TypeError:     # an unhashable constexpr: the Python path reports it
@@ -460,11 +473,7 @@ class JITFunction:
                 self._fast[csig] = fast
         ck, values = fast
         if callable(grid):
-            meta = dict(self.defaults)
-            meta.update(zip(self.param_names, args))
-            meta.update(kwargs)
-            meta["num_warps"] = num_warps
-            grid = grid(meta)
+            grid = self._grid_of(grid, args, {**kwargs, "num_warps": num_warps})
         if type(grid) is not tuple:
             grid = (grid,) if isinstance(grid, int) else tuple(grid)
         if len(grid) == 1:
