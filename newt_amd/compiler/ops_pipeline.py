@@ -431,47 +431,60 @@ class DotPipeline:
         state["pf"] = {}
         state["late"] = []
         self.pipe_records.append(state)
+        ctx = (node, state, S, n, lo_e, stv, idt, slice_stmts, advance, skip, temps, kname, flat)
+        state["clamp"] = os.environ.get("NEWT_PIPE_CLAMP", "1") != "0"
+        versioned = plan["fast_ok"] and os.environ.get("NEWT_PIPE_VERSION", "1") != "0"
+        state["bufdma"] = versioned and os.environ.get("NEWT_BUFFER_DMA", "1") != "0"
+        ahead = self._plan_ahead(ctx) if state["bufdma"] else None
         for s in range(S - 1):
             self.locals[kname] = self.new_scalar(idt, f"({lo_e} + {s * stv})")
             self.visit_body(slice_stmts)
+            if ahead:
+                self._ahead_prologue(state, s)
             self.pipe_issue(state, s, f"({s} < {n.expr})")
+            if ahead:
+                self.indent -= 1
+                self.emit("}")
             self.visit_body(advance)
             for t in temps:
                 self.locals.pop(t, None)
+        if ahead:
+            self.emit(f"if ({ahead['go']}) {{")
+            self.indent += 1
+            for test, ahead["edge"] in ahead["modes"]:
+                self.emit(f"{test} {{")
+                self._ahead_write(state, 0)
+                self.emit("}")
+            self.indent -= 1
+            self.emit("}")
         self.pipe_hoist_operands(state)
         rec = self._enter_compound(node)
         self.drain_dots_for_loop(node)
         it0 = self.fresh("it")
         self.emit(f"{idt.ctype} {it0} = 0;")
         mark = len(self.lines)
-        ctx = (node, state, S, n, lo_e, stv, idt, slice_stmts, advance, skip, temps, kname, flat)
-        state["clamp"] = os.environ.get("NEWT_PIPE_CLAMP", "1") != "0"
-        state["clamp_n"] = n
-        if plan["fast_ok"] and os.environ.get("NEWT_PIPE_VERSION", "1") != "0":
+        if versioned:
             state["fast_emitted"] = True
             # leading iterations whose every tile is a whole in-bounds copy run
             # in a copy of the loop with no per-iteration tests at all; its
             # copies take the buffer form (32-bit lane offsets) when every
             # tile's lane offsets fit, which joins the entry test
-            state["bufdma"] = os.environ.get("NEWT_BUFFER_DMA", "1") != "0"
-            nf = self._fast_count(ctx)
-            self.emit(f"for (; {it0} + {2 * S - 2} < {nf.expr}; {it0} += {S}) {{")
-            self._pipe_iterations(ctx, it0, fast=True)
-            self.emit("}")
-            if state["clamp"]:
-                # when every iteration is fast, one more branch-free trip runs
-                # S of the last iterations: its copies past the end repeat the
-                # last tile into stages no iteration reads again, so every
-                # sub-iteration keeps the same copies in flight and the same
-                # waits (the general loop ran these ~1.5x slower). The loop
-                # above stays as it was: clamping there lengthened the scalar
-                # work ahead of every copy.
-                self.emit(f"if ((({nf.expr}) == ({n.expr})) && {it0} + {S - 1} < {n.expr}) {{")
-                state["clamp_trip"] = True
-                self._pipe_iterations(ctx, it0, fast=True)
-                state["clamp_trip"] = False
-                self.emit(f"  {it0} += {S};")
+            if ahead:
+                self.emit(f"if ({ahead['go']}) {{")
+                self.indent += 1
+                for test, mode in ahead["modes"]:
+                    self.emit(f"{test} {{")
+                    self.indent += 1
+                    ahead["edge"] = mode
+                    self._fast_loops(ctx, it0, ahead["nf"])
+                    for d in range(1, S - 1):
+                        self._ahead_write(state, d)
+                    self.indent -= 1
+                    self.emit("}")
+                self.indent -= 1
                 self.emit("}")
+            else:
+                self._fast_loops(ctx, it0, self._fast_count(ctx))
         self.emit(f"for (; {it0} < {n.expr}; {it0} += {S}) {{")
         self._pipe_iterations(ctx, it0, fast=False)
         self.emit("}")
@@ -488,6 +501,222 @@ class DotPipeline:
         self.after_loop(node)
         if state["recs"] is not None:
             self.lds_pool.extend(state["lds_idx"])
+
+    def _fast_loops(self, ctx, it0, nf):
+        """The branch-free copy of the loop over its leading fast iterations."""
+        state, S, n = ctx[1], ctx[2], ctx[3]
+        self.emit(f"for (; {it0} + {2 * S - 2} < {nf.expr}; {it0} += {S}) {{")
+        self._pipe_iterations(ctx, it0, fast=True)
+        self.emit("}")
+        if state["clamp"]:
+            # when every iteration is fast, one more branch-free trip runs
+            # S of the last iterations: its copies past the end repeat the
+            # last tile into stages no iteration reads again, so every
+            # sub-iteration keeps the same copies in flight and the same
+            # waits (the general loop ran these ~1.5x slower). The loop
+            # above stays as it was: clamping there lengthened the scalar
+            # work ahead of every copy.
+            self.emit(f"if ((({nf.expr}) == ({n.expr})) && {it0} + {S - 1} < {n.expr}) {{")
+            state["clamp_trip"] = True
+            self._pipe_iterations(ctx, it0, fast=True)
+            state["clamp_trip"] = False
+            self.emit(f"  {it0} += {S};")
+            self.emit("}")
+
+    # ------------------------------------- tiles loaded several iterations ahead
+    def _plan_ahead(self, ctx):
+        """Decide whether the branch-free loop loads its tiles into registers
+        S-1 iterations ahead, and set it up; None where copies go straight to
+        LDS or a tile does not allow it.
+
+        A tile that cannot be copied straight to LDS (rows of an odd stride)
+        is loaded into VGPRs and written to LDS from there. One iteration's
+        MFMAs do not cover a load's latency, so iteration i loads the tile of
+        i+S-1 into one of S register sets and writes that of i+1 to its stage.
+        Loads are unconditional 16-byte buffer loads: a chunk outside an
+        unchanging row mask takes an offset past the descriptor's range and
+        reads as zeros. A program whose column bound cuts a chunk runs another
+        copy of the loop, in which that chunk is read so that it ends at the
+        bound and shifted into place on its way to LDS, or, where the bound
+        lies inside the tile's first chunk, one with a load per element (a
+        branch between two loads of one register would drain every load in
+        flight). Tiles
+        that could be copied straight to LDS are loaded the same way: the
+        mixture would count register loads among the copies it waits for.
+        fp16 1000x1003x777 15.1 -> 10.2 us (64x64x64 on 8 waves, 3
+        stages; x @ w.t() 12.3 -> 9.4), 2048x2047x2049 72 -> 32.6 (128x128x32 on
+        8 waves; the one-iteration form was slower there than 64x64 tiles).
+        With a load per element in every edge program, which the launch waits
+        for, the two ran 16.4 and 72.8."""
+        node, state, S, n, lo_e, stv, idt, slice_stmts, advance, skip, temps, kname, flat = ctx
+        state["ahead"] = None
+        self.locals[kname] = self.new_scalar(idt, lo_e)
+        self.visit_body(slice_stmts)
+        if state["recs"] is None:
+            self._init_recs(state)
+        regs = 0
+        ok = state["acc_name"] is not None
+        for r in state["recs"].values():
+            X = self.locals[r["name"]]
+            V = X if r["kdim"] == 1 else self.permute(X, (1, 0))
+            ok = ok and self._ahead_tile(r, X, V, state["plan"])
+            regs += r["R"] * r["K"] * r["dt"].itemsize // 4 // self.T
+            for ld in (X, V):
+                ld.consumed = True
+                if ld in self.pending_loads:
+                    self.pending_loads.remove(ld)
+        for t in temps:
+            self.locals.pop(t, None)
+        tiles = [r["R"] for r in state["recs"].values()]
+        # the register sets and the accumulators share 256 VGPRs with the rest
+        if (not ok or all(r["dma"] for r in state["recs"].values()) or len(tiles) != 2
+                or math.prod(tiles) // self.T + S * regs > 160):
+            return None
+        state["plr"] = False
+        ahead = state["ahead"] = {"edge": "", "sets": []}
+        # how a column bound meets the tile: not at all, at or past its first
+        # whole chunk, or inside it
+        edged = [r for r in state["recs"].values() if r["edge"]]
+        ahead["modes"] = [("", "")]
+        if edged:
+            whole = " && ".join(f"({r['edge_full']})" for r in edged)
+            shift = " && ".join(f"({r['bound']} <= -{16 // r['dt'].itemsize} || {r['bound']} >= 0)"
+                                for r in edged)
+            ahead["modes"] = [(f"if ({whole})", ""), (f"else if ({shift})", "shift"),
+                              ("else", "each")]
+        nf = self._fast_count(ctx)
+        ahead["nf"] = nf
+        ahead["go"] = self.new_scalar(tp.int1, f"({2 * S - 2} < {nf.expr})").expr
+        for s in range(S):
+            regs = {}
+            for r in state["recs"].values():
+                var = self.fresh("ra")
+                self.emit(f"u32x4 {var}[{r['layout'].nslots // (16 // r['dt'].itemsize)}];")
+                regs[r["name"]] = var
+            ahead["sets"].append(regs)
+        return ahead
+
+    def _ahead_tile(self, r, X, V, plan):
+        """Whether a tile can be loaded ahead; records its register layout and
+        the mask comparisons that no iteration changes."""
+        epc = 16 // r["dt"].itemsize
+        cdim = 1 if r["fmt"] == "k" else 0
+        off = V.ptr.offset
+        if not isinstance(off, Affine) or X.dtype != r["dt"]:
+            return False
+        L = (self.staging_layout(V) if cdim == 1
+             else lo.blocked((r["K"], r["R"]), self.W, min(epc, r["R"])).permute((1, 0)))
+        # runs along the dim that is contiguous in LDS (a K-major tile may be
+        # contiguous along its rows in memory: 16 rows have no R-major form)
+        if (L.reg[0] is None or L.reg[0][0] != cdim or (1 << self.contiguous_bits(L, off)) < epc
+                or L.nslots % epc or self.canon_cond(L)):
+            return False
+        r["layout"], r["unchanging"], r["edge"] = L, (), ()
+        if V.mask is None:
+            return True
+        meta = getattr(V.mask, "meta", None) if isinstance(V.mask, Lazy) else None
+        other = X.other.value if isinstance(X.other, Fill) else X.other
+        if not meta or not (other is None or (isinstance(other, Const) and other.pyval == 0)):
+            return False
+        call = plan["flat"][plan["staged"][r["name"]]["index"]].value
+        masks = [k.value for k in call.keywords if k.arg == "mask"] + list(call.args[1:2])
+        forms = self._mask_forms(masks[0], plan)
+        if forms is None or len(forms) != len(meta[1]) or self.mask_all_true(V.mask, V.shape) is None:
+            return False
+        r["unchanging"] = tuple(i for i, f in enumerate(forms) if f == "c")
+        one = Lazy(tp.int1, V.shape, None, [])
+        for i in r["unchanging"]:
+            one.meta = ("and", [meta[1][i]])
+            if self.chunk_mask(one, cdim, epc) is None:
+                r["edge"] += (i,)
+        if r["edge"]:
+            # one bound `base + column < 0` on the contiguous dim
+            _, sym, aff = meta[1][r["edge"][0]]
+            c = [(d, v) for d, v in aff.coefs.items() if aff.shape[d] > 1]
+            if (len(r["edge"]) > 1 or sym != "<" or aff.dtype != tp.int32 or len(c) != 1
+                    or c[0][0] != cdim or not c[0][1].is_const or c[0][1].const != 1):
+                return False
+            r["bound"] = self.new_scalar(tp.int32, aff.base.expr).expr
+            r["edge_full"] = self.mask_all_true(V.mask, V.shape, set(r["edge"]))
+        return True
+
+    def _ahead_load(self, state, s, edge):
+        """Load the tiles of the slice just visited into register set s."""
+        for r in state["recs"].values():
+            X = self.locals[r["name"]]
+            V = X if r["kdim"] == 1 else self.permute(X, (1, 0))
+            dt, L = r["dt"], r["layout"]
+            epc = 16 // dt.itemsize
+            cdim = 1 if r["fmt"] == "k" else 0
+            off, base = V.ptr.offset, V.ptr.base.expr
+            if not (off.base.is_const and off.base.const == 0):
+                base = f"({base} + ({off.base.expr}))"
+            each, shift = r["edge"] and edge == "each", r["edge"] and edge == "shift"
+            parts = [V.mask.meta[1][i] for i in r["unchanging"] if each or i not in r["edge"]]
+            for g in range(0, L.nslots, epc):
+                at = (self.coord(L, 0, g), self.coord(L, 1, g))
+                lane = " + ".join(x if c.is_const and c.const == 1 else f"{c.expr} * {x}"
+                                  for c, x in ((off.coefs.get(d), at[d]) for d in (0, 1))
+                                  if c is not None) or "0"
+                ok = self.mask_expr(parts, at)
+                if shift:
+                    # the chunk that the bound cuts is read so that it ends there
+                    lane = f"{lane} - newt::run_past({r['bound']} + {at[cdim]} + {epc})"
+                    ok = f"{ok} && {r['bound']} + {at[cdim]} < 0"
+                lane = f"(unsigned)(({lane}) * {dt.itemsize})"
+                dst = f"{state['ahead']['sets'][s][r['name']]}[{g // epc}]"
+                if each:
+                    ins = []
+                    for i in range(epc):
+                        x = list(at)
+                        x[cdim] = f"({at[cdim]} + {i})"
+                        ins.append(self.mask_expr(parts, x))
+                    self.emit(f"{{ const bool _m[{epc}] = {{{', '.join(ins)}}}; {dst} = "
+                              f"newt::buf_load16_each<{dt.ctype}>({base}, {lane}, _m); }}")
+                else:
+                    self.emit(f"{dst} = newt::buf_load16({base}, {lane}, {ok});")
+            for ld in (X, V):
+                ld.consumed = True
+                if ld in self.pending_loads:
+                    self.pending_loads.remove(ld)
+
+    def _ahead_prologue(self, state, s):
+        """Tile s, for the branch-free loop into register set s; else (the
+        caller closes that branch) as the general loop expects it."""
+        ahead = state["ahead"]
+        names = [r["name"] for r in state["recs"].values()]
+        saved = {nm: self.locals[nm] for nm in names}
+        self.emit(f"if ({ahead['go']}) {{")
+        self.indent += 1
+        for test, mode in ahead["modes"]:
+            self.emit(f"{test} {{")
+            self._ahead_load(state, s, mode)
+            self.emit("}")
+            for nm, X in saved.items():
+                self.locals[nm] = X
+        self.indent -= 1
+        self.emit("} else {")
+        self.indent += 1
+        for nm, X in saved.items():
+            X.consumed = False
+            self.locals[nm] = X
+
+    def _ahead_write(self, state, s):
+        """Write register set s to stage s."""
+        for r in state["recs"].values():
+            L, dt = r["layout"], r["dt"]
+            epc = 16 // dt.itemsize
+            T = dt.ctype
+            for g in range(0, L.nslots, epc):
+                rr, kk = self.coord(L, 0, g), self.coord(L, 1, g)
+                o = (f"newt::LdsTile<{T}, {r['K']}>::off({rr}, {kk})" if r["fmt"] == "k"
+                     else f"newt::LdsTileR32<{r['R']}>::off({kk}, {rr})" if dt == tp.float32
+                     else f"newt::LdsTileR<{T}, {r['R']}, {r['sb']}>::off({kk}, {rr})")
+                v = f"{state['ahead']['sets'][s][r['name']]}[{g // epc}]"
+                if r["edge"] and state["ahead"]["edge"] == "shift":
+                    c = kk if r["fmt"] == "k" else rr
+                    v = f"newt::drop_low<{T}>({v}, newt::run_past({r['bound']} + {c} + {epc}))"
+                self.emit(f"*(u32x4*)(({T}*)({state['names'][s]} + {r['off']}) + {o}) = {v};")
 
     def _insert_lines(self, index, lines):
         ind = "  " * self.indent
@@ -692,7 +921,19 @@ class DotPipeline:
             X = self.locals.get(r["name"])
             if not isinstance(X, LazyLoad) or X.result is not None or tuple(X.shape) != r["shape"]:
                 self._no_pipe(state)
-            if r["dma"]:
+            if state.get("ahead"):
+                V = X if r["kdim"] == 1 else self.permute(X, (1, 0))
+                parts = None
+                if r["unchanging"]:
+                    parts = set(range(len(V.mask.meta[1]))) - set(r["unchanging"])
+                full = self.mask_all_true(V.mask, V.shape, parts)
+                if full != "true":
+                    conds.append(f"({full})")
+                conds.append(f"({self._lane_bytes_fit(V, r['R'], r['K'], r['dt'])})")
+                V.consumed = True
+                if V in self.pending_loads:
+                    self.pending_loads.remove(V)
+            elif r["dma"]:
                 # comparisons that no iteration changes are left to the copies
                 parts = None
                 if r["inv"] and state.get("bufdma"):
@@ -731,7 +972,9 @@ class DotPipeline:
             # with prefetching, iteration it+1 must also have landed: its first
             # k-step is read before the next barrier
             deep = (S - 3 if plr else S - 2) * ops
-            if deep and fast:
+            if fast and state.get("ahead"):
+                pass    # no copies in flight: LDS is written from registers
+            elif deep and fast:
                 self.emit(f"newt::wait_vmcnt<{deep}>();")
             elif deep:
                 self.emit(f"if ({it} + {S - 2} < {n.expr}) newt::wait_vmcnt<{deep}>(); "
@@ -757,7 +1000,12 @@ class DotPipeline:
             else:
                 self.locals[kname] = self.new_scalar(idt, f"({lo_e} + {issue} * {stv})")
             self.visit_body(slice_stmts)
-            self.pipe_issue(state, (s + S - 1) % S, f"({issue} < {n.expr})", fast=fast)
+            ahead = state.get("ahead") if fast else None
+            if ahead:
+                self._ahead_load(state, (s + S - 1) % S, ahead["edge"])
+                self.emit("__builtin_amdgcn_sched_barrier(0);")
+            else:
+                self.pipe_issue(state, (s + S - 1) % S, f"({issue} < {n.expr})", fast=fast)
             if clamp and advance:
                 self.emit(f"if ({issue} < {n.expr} - 1) {{")
                 self.indent += 1
@@ -779,9 +1027,12 @@ class DotPipeline:
                 self.locals.pop(t, None)
             if plr:
                 self._plr_fill(state, (s + 1) % S)
-            if fast:
+            if ahead:
+                self.emit("__builtin_amdgcn_sched_barrier(0);")
+                self._ahead_write(state, (s + 1) % S)
+            elif fast:
                 self._write_late(state)
-            if fast and state["simple"] and os.environ.get("NEWT_SCHED", "1") != "0":
+            if fast and not ahead and state["simple"] and os.environ.get("NEWT_SCHED", "1") != "0":
                 self._sched_hints(state)
         self.pipe_active = None
         self.flush_loads()
@@ -1097,10 +1348,10 @@ class DotPipeline:
         """Write the register-path tiles that the branch-free loop loaded
         before its MFMAs into their stage: no wave reads that stage again
         before the next iteration's barrier, which also publishes it. Bound by
-        the load latency that one iteration's MFMAs do not cover. With 16-byte
-        loads at any alignment, fp16 1000x1003x777 (odd strides) takes 13.7 us
-        against 25.2 for the same tile with 2-byte loads waited for at once,
-        2048x2047x2049 72 against 149; aligned 1024x1024x768 takes 5.9."""
+        the load latency that one iteration's MFMAs do not cover; loops that
+        _plan_ahead does not take run this. With 16-byte loads at any
+        alignment, fp16 1000x1003x777 (odd strides) took 13.7 us this way
+        against 25.2 for the same tile with 2-byte loads waited for at once."""
         late, state["late"] = state["late"], []
         if late:
             self.emit("__builtin_amdgcn_sched_barrier(0);")

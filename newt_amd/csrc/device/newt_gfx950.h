@@ -709,6 +709,54 @@ __device__ __forceinline__ void lds_copy16_if(const void* g, bool in, void* dst)
   *(u32x4*)dst = v;
 }
 
+// 16 bytes at base + lane_bytes into registers where `in` holds, zeros elsewhere
+// (the range check, as above), with no branch, so the loads of several
+// iterations stay in flight together. Any element alignment.
+__device__ __forceinline__ u32x4 buf_load16(const void* base, unsigned lane_bytes, bool in) {
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<void*>(base), (short)0, (int)0x80000000, 0x00020000);
+  return __builtin_amdgcn_raw_buffer_load_b128(rs, in ? lane_bytes : 0x80000000u, 0, 0);
+}
+
+// The same 16 bytes one element at a time, each under its own condition.
+template <typename T>
+__device__ __forceinline__ u32x4 buf_load16_each(const void* base, unsigned lane_bytes,
+                                                 const bool* in) {
+  static_assert(sizeof(T) == 2 || sizeof(T) == 4, "16- and 32-bit elements");
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<void*>(base), (short)0, (int)0x80000000, 0x00020000);
+  u32x4 v;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (sizeof(T) == 4) {
+      v[i] = __builtin_amdgcn_raw_buffer_load_b32(rs, in[i] ? lane_bytes + 4 * i : 0x80000000u, 0, 0);
+    } else {
+      const u32 a = __builtin_amdgcn_raw_buffer_load_b16(
+          rs, in[2 * i] ? lane_bytes + 4 * i : 0x80000000u, 0, 0);
+      const u32 b = __builtin_amdgcn_raw_buffer_load_b16(
+          rs, in[2 * i + 1] ? lane_bytes + 4 * i + 2 : 0x80000000u, 0, 0);
+      v[i] = a | b << 16;
+    }
+  }
+  return v;
+}
+
+// Elements by which a run of N that starts at `past - N` before a bound reaches
+// past it (none when past <= 0).
+__device__ __forceinline__ int run_past(int past) { return past > 0 ? past : 0; }
+
+// The 16 bytes v with its n lowest elements dropped, zeros shifted in above
+// (0 <= n < 16 / sizeof(T); any value for n beyond that range).
+template <typename T>
+__device__ __forceinline__ u32x4 drop_low(u32x4 v, int n) {
+  const int bits = n * 8 * (int)sizeof(T);
+  const u32x4 a = bits & 32 ? u32x4{v[1], v[2], v[3], 0u} : v;
+  const u32x4 b = bits & 64 ? u32x4{a[2], a[3], 0u, 0u} : a;
+  return u32x4{__builtin_amdgcn_alignbit(b[1], b[0], bits & 31),
+               __builtin_amdgcn_alignbit(b[2], b[1], bits & 31),
+               __builtin_amdgcn_alignbit(b[3], b[2], bits & 31), b[3] >> (bits & 31)};
+}
+
 // Wait until at most N vector-memory operations of this wave are outstanding
 // (s_waitcnt vmcnt(N); expcnt and lgkmcnt left unconstrained).
 template <int N>

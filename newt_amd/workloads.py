@@ -199,9 +199,11 @@ MATMUL_CONFIGS = [
     # two waves per SIMD over a 64x128 tile: bf16 640x2048x2048 (320 such
     # tiles) 12.7 us against 15.1 for 64x64x64 and 15.5 for 128x128x64
     newt.Config({"BLOCK_M": 64, "BLOCK_N": 128, "BLOCK_K": 64}, num_warps=8, num_stages=4),
-    # odd strides: tiles that go through registers want few bytes per wave and
-    # several workgroups per CU (fp16 1024x1025x1152: 8 waves and 2 stages)
-    newt.Config({"BLOCK_M": 64, "BLOCK_N": 64, "BLOCK_K": 64}, num_warps=8, num_stages=2),
+    # odd strides: tiles that go through registers want few bytes per wave
+    # (fp16 2048x2047x2049 32.6 us against 37.1 on 4 waves and 48.6 on 64x64
+    # tiles; 1000x1003x777 10.2 against 11.8 on 4 waves)
+    newt.Config({"BLOCK_M": 128, "BLOCK_N": 128, "BLOCK_K": 32}, num_warps=8, num_stages=4),
+    newt.Config({"BLOCK_M": 64, "BLOCK_N": 64, "BLOCK_K": 64}, num_warps=8, num_stages=3),
 ]
 
 matmul_tuned = newt.autotune(configs=MATMUL_CONFIGS, key=["M", "N", "K"])(matmul_kernel)
@@ -231,7 +233,7 @@ MATMUL_CONFIGS_SMALL = [
     newt.Config({"BLOCK_M": 64, "BLOCK_N": 64, "BLOCK_K": 64}, num_warps=4, num_stages=4),
     newt.Config({"BLOCK_M": 64, "BLOCK_N": 64, "BLOCK_K": 128}, num_warps=4, num_stages=4),
     newt.Config({"BLOCK_M": 64, "BLOCK_N": 32, "BLOCK_K": 64}, num_warps=4, num_stages=4),
-    newt.Config({"BLOCK_M": 64, "BLOCK_N": 64, "BLOCK_K": 64}, num_warps=8, num_stages=2),
+    newt.Config({"BLOCK_M": 64, "BLOCK_N": 64, "BLOCK_K": 64}, num_warps=8, num_stages=3),
 ]
 matmul_tuned_small = newt.autotune(configs=MATMUL_CONFIGS_SMALL,
                                    key=["M", "N", "K"])(matmul_kernel)

@@ -88,10 +88,18 @@ def test_fp32_masked_copies():
 @pytest.mark.parametrize("tile", [(64, 64, 64, 8, 2), (64, 64, 64, 4, 4), (128, 128, 32, 4, 3),
                                   (32, 64, 128, 4, 2)])
 @pytest.mark.parametrize("lda,ldb", [(1033, 64), (1040, 65), (1033, 67)])
-@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (13, 9, 65), (31, 63, 1032), (64, 64, 1024)])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (13, 9, 65), (31, 63, 1032), (64, 64, 1024),
+                                   (63, 7, 700), (64, 8, 832), (5, 15, 513)])
 def test_odd_strides(tile, lda, ldb, M, N, K):
-    """Rows of an odd stride: tiles loaded into registers at their elements'
-    alignment ahead of the MFMAs and written to LDS after them, beside tiles
-    that are copied asynchronously."""
+    """Rows of an odd stride: tiles loaded into registers several iterations
+    ahead at their elements' alignment, whole, cut by the column bound after
+    their first chunk (shifted into place) or inside it (element loads), over
+    trip counts from none in the branch-free loop to several."""
     BM, BN, BK, waves, stages = tile
     case(min(M, BM), min(N, BN), K, lda, ldb, BM, BN, BK, waves, stages)
+
+
+@pytest.mark.parametrize("N", [9, 60, 61, 62, 63])
+def test_odd_strides_fp32(N):
+    """32-bit elements: four to a chunk, bounds that cut one to three off."""
+    case(61, N, 260, 261, 67, 64, 64, 16, 4, 4, dtype=torch.float32)
