@@ -32,6 +32,8 @@ reference's examples/01-05), extended to the benchmark configurations:
 Everything is compiled by newt_amd's compiler to HIP for gfx950.
 """
 
+import functools
+
 import torch
 
 import newt_amd as newt
@@ -486,38 +488,51 @@ def attention_plain_kernel(q_ptr, k_ptr, v_ptr, o_ptr, S, H, scale,
     nl.store(o_base + offs_m[:, None] * som + offs_d[None, :], acc, mask=qmask)
 
 
+@functools.lru_cache(maxsize=1024)
 def attention_tile(S, heads, D, causal):
     """(query rows, waves) of a program of the default kernel at 64-key blocks.
 
-    256 rows on 8 waves share each K and V block between the most rows, but a
-    launch needs programs for 256 CUs. Smaller tiles of 16 rows per wave keep
-    4 or 8 waves on a CU's four SIMDs; they read K and V from LDS more often
-    per row, which costs a launch that fills the chip anyway 15-24% at head
-    dim 128 and 3-7% at 64 (where 128 rows on 4 waves run 1-2% ahead of 256).
-    Not causal: the tile with the least rows on the busiest CU, weighed by
-    those rates: bf16 [1,16,1000,128] 32.0 us on 256 rows, 22.4 on 128, 18.5
-    on 64; [1,8,4096,128] 100.9 / 75.2 / 85.9; [2,32,4096,128] 444 / 540 / 583;
-    fp16 [2,16,1000,64] 23.9 / 17.2 / 17.9; bf16 [3,8,1500,64] 32.6 / 32.3 /
-    28.9. Causal: programs differ in length (the last query block attends to
-    every key), so a tile also wants several programs per CU:
-    [2,32,2048,128] 76.7 / 89.8 / 91.8 (512 programs of 256 rows),
-    [1,32,2048,128] 57.9 / 45.6 / 50.3 (256), [1,8,4096,128] 97.4 / 66.5 /
-    59.3; [4,32,2048,64] 110.7 / 105.9 / 104.6, [2,16,2048,64] 42.6 / 32.4 /
-    30.7."""
-    wide = D > 64
-    programs = {rows: newt.cdiv(S, rows) * heads for rows in (256, 128, 64)}
-    waves = {256: 8, 128: 8 if wide else 4, 64: 4}
-    if causal:
-        if wide and programs[256] >= 512:
-            rows = 256
-        elif programs[128] >= (512 if wide else 1024):
-            rows = 128
+    256 rows on 8 waves share each K and V block between the most rows, but
+    one such workgroup takes a whole CU: a launch wants a multiple of 256 of
+    them. 128 rows on 4 waves run two to a CU, in half the steps and 2-6%
+    slower per row (1-2% faster at head dim 64); 128 rows on 8 waves and 64 on
+    4 keep 16 rows per wave and so read K and V twice as often, which costs
+    15-25% where the chip is full anyway but fills four SIMDs with the fewest
+    rows. Lines drawn from bf16 sweeps of 256 to 4096 keys over 96 to 1024
+    programs of 256 rows (us, [heads, S]; 256x8 / 128x8 / 128x4 / 64x4):
+      not causal, D 128: [24, 1024] 30.7 / 21.1 / 22.1 / 22.7, [40, 1024] 31.4 /
+      39.7 / 34.1 / 35.0, [68, 1024] 63.0 / 58.8 / 52.8 / 53.8, [100, 1024] 63.6 /
+      79.1 / 66.7 / 73.0: the costs below are rounds of the 256 CUs, measured in
+      full rounds of 256 rows;
+      causal, D 128 (the programs of a head differ in length, so more of them
+      also balance better): [32, 1024] 33.4 / 22.0 / 24.3 / 18.8, [64, 1024] 35.6 /
+      29.7 / 36.6 / 31.8, [112, 1024] 52.9 / 57.5 / 49.7 / 52.0, [40, 2048] 58.7 /
+      62.4 / 52.2 / 59.8, [64, 2048] 76.1 / 87.4 / 80.0 / 90.0, [80, 2048] 104 / 114 /
+      96 / 112, [128, 2048] 166 / 188 / 168 / 192;
+      causal, D 64: [64, 1024] 24.3 / 24.2 / 23.6 / 20.2, [256, 1024] 74.2 / 64.2 /
+      60.7 / 58.7, [64, 2048] 52.1 / 53.9 / 50.0 / 55.9, [32, 2048] 41.9 / 32.6 /
+      30.1 / 28.3."""
+    def rounds(rows):
+        return newt.cdiv(newt.cdiv(S, rows) * heads, 256)
+
+    programs = newt.cdiv(S, 256) * heads
+    if not causal:
+        if D > 64:
+            cost = {(256, 8): 0.88 * rounds(256) + 0.02, (128, 8): 0.58 * rounds(128),
+                    (128, 4): max(0.45 * rounds(128) + 0.1, 0.61),
+                    (64, 4): 0.29 * rounds(64) + 0.06}
         else:
-            rows = 64
-    else:
-        rate = {256: 1.0, 128: 0.85, 64: 0.78} if wide else {256: 1.0, 128: 1.02, 64: 0.93}
-        rows = min(rate, key=lambda r: newt.cdiv(programs[r], 256) * r / rate[r])
-    return rows, waves[rows]
+            cost = {(256, 8): rounds(256), (128, 4): rounds(128) / 2.04,
+                    (64, 4): rounds(64) / 3.72}
+        return min(cost, key=cost.get)
+    if D <= 64:
+        return (64, 4) if S <= 1024 or rounds(128) < 4 else (128, 4)
+    if programs <= 256:
+        return (128, 8) if programs > 160 and S > 512 else (64, 4)
+    # long sequences: one and a half, two, and from four rounds on 256 rows win
+    if S >= 2048 and (programs >= 1024 or programs in (384, 512)):
+        return 256, 8
+    return 128, 4
 
 
 def attention(q, k, v, causal=False, scale=None, out=None, BLOCK_M=None, BLOCK_N=64,
@@ -544,31 +559,17 @@ def attention(q, k, v, causal=False, scale=None, out=None, BLOCK_M=None, BLOCK_N
         BLOCK_M = 256
     if num_warps is None:
         num_warps = BLOCK_M // 32
-    for t in (q, k, v):
-        if t.stride(3) != 1:
-            raise ValueError("attention: q, k and v need unit stride along head_dim")
     out = torch.empty_like(q) if out is None else out
-    if out.stride(3) != 1:
+    sq, sk, sv, so = q.stride(), k.stride(), v.stride(), out.stride()
+    if not sq[3] == sk[3] == sv[3] == 1:
+        raise ValueError("attention: q, k and v need unit stride along head_dim")
+    if so[3] != 1:
         raise ValueError("attention: out needs unit stride along head_dim")
-    grid = (newt.cdiv(S, BLOCK_M), B * H)
-    if plain:
-        attention_plain_kernel[grid](q, k, v, out, S, H, scale,
-                                     q.stride(0), q.stride(1), q.stride(2),
-                                     k.stride(0), k.stride(1), k.stride(2),
-                                     v.stride(0), v.stride(1), v.stride(2),
-                                     out.stride(0), out.stride(1), out.stride(2),
-                                     BLOCK_M=BLOCK_M, BLOCK_N=BLOCK_N, D=D, CAUSAL=causal,
-                                     num_warps=num_warps, num_stages=num_stages,
-                                     waves_per_eu=waves_per_eu)
-        return out
-    attention_kernel[grid](q, k, v, out, S, H, scale,
-                           q.stride(0), q.stride(1), q.stride(2),
-                           k.stride(0), k.stride(1), k.stride(2),
-                           v.stride(0), v.stride(1), v.stride(2),
-                           out.stride(0), out.stride(1), out.stride(2),
-                           BLOCK_M=BLOCK_M, BLOCK_N=BLOCK_N, D=D, CAUSAL=causal,
-                           num_warps=num_warps, num_stages=num_stages,
-                           waves_per_eu=waves_per_eu)
+    kernel = attention_plain_kernel if plain else attention_kernel
+    kernel[(newt.cdiv(S, BLOCK_M), B * H)](
+        q, k, v, out, S, H, scale, *sq[:3], *sk[:3], *sv[:3], *so[:3],
+        BLOCK_M=BLOCK_M, BLOCK_N=BLOCK_N, D=D, CAUSAL=causal, num_warps=num_warps,
+        num_stages=num_stages, waves_per_eu=waves_per_eu)
     return out
 
 

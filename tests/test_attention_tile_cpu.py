@@ -7,16 +7,21 @@ from newt_amd.workloads import attention_tile
 
 @pytest.mark.parametrize("S,heads,D,causal,want", [
     (4096, 128, 128, True, (256, 8)), (4096, 128, 128, False, (256, 8)),
-    # causal, wide heads: 512 programs of 256 rows, then 512 of 128
-    (2048, 64, 128, True, (256, 8)), (2048, 63, 128, True, (128, 8)),
-    (2048, 32, 128, True, (128, 8)), (2048, 31, 128, True, (64, 4)),
-    # causal, 64-wide heads: 1024 programs of 128 rows
-    (2048, 64, 64, True, (128, 4)), (2048, 63, 64, True, (64, 4)),
-    # not causal: 193 programs of 256 rows, then 129 to 256 of 128
-    (256, 193, 128, False, (256, 8)), (256, 192, 128, False, (64, 4)),
-    (256, 128, 128, False, (128, 8)), (256, 65, 128, False, (128, 8)),
-    (256, 64, 128, False, (64, 4)), (1, 1, 128, False, (64, 4)),
-    (1000, 32, 64, False, (128, 4)), (1500, 24, 64, False, (64, 4)),
+    # causal, wide heads: 160, 256, 512 and 1024 programs of 256 rows
+    (1024, 40, 128, True, (64, 4)), (1024, 41, 128, True, (128, 8)),
+    (512, 128, 128, True, (64, 4)), (2048, 32, 128, True, (128, 8)),
+    (2048, 33, 128, True, (128, 4)), (2048, 64, 128, True, (256, 8)),
+    (2048, 65, 128, True, (128, 4)), (2048, 48, 128, True, (256, 8)), (2048, 128, 128, True, (256, 8)),
+    (1024, 256, 128, True, (128, 4)),
+    # causal, 64-wide heads: 1024 keys, then 768 programs of 128 rows
+    (1024, 256, 64, True, (64, 4)), (2048, 48, 64, True, (64, 4)),
+    (2048, 49, 64, True, (128, 4)),
+    # not causal: rounds of the 256 CUs
+    (256, 256, 128, False, (256, 8)), (256, 129, 128, False, (256, 8)),
+    (256, 128, 128, False, (128, 8)), (256, 257, 128, False, (128, 4)),
+    (256, 400, 128, False, (256, 8)), (256, 64, 128, False, (64, 4)),
+    (1, 1, 128, False, (64, 4)), (1000, 32, 64, False, (128, 4)),
+    (1500, 24, 64, False, (64, 4)),
 ])
 def test_tile_rule(S, heads, D, causal, want):
     assert attention_tile(S, heads, D, causal) == want
