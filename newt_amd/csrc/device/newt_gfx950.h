@@ -718,6 +718,14 @@ __device__ __forceinline__ u32x4 buf_load16(const void* base, unsigned lane_byte
   return __builtin_amdgcn_raw_buffer_load_b128(rs, in ? lane_bytes : 0x80000000u, 0, 0);
 }
 
+template <typename T, int N>
+__device__ __forceinline__ void buf_load_vec(const T* base, unsigned lane_bytes, bool in, T* out) {
+  static_assert(sizeof(T) * N == 16, "one 16-byte run");
+  vec_t<T, N> v = __builtin_bit_cast(vec_t<T, N>, buf_load16(base, lane_bytes, in));
+#pragma unroll
+  for (int i = 0; i < N; ++i) out[i] = v.d[i];
+}
+
 // The same 16 bytes one element at a time, each under its own condition.
 template <typename T>
 __device__ __forceinline__ u32x4 buf_load16_each(const void* base, unsigned lane_bytes,

@@ -32,7 +32,8 @@ def copy_prefix_k(x_ptr, o_ptr, N, stride, BLOCK: nl.constexpr):
 @pytest.mark.parametrize("dtype", [torch.int8, torch.float16, torch.float32, torch.int64])
 @pytest.mark.parametrize("offset", [0, 1, 3])
 @pytest.mark.parametrize("N,first,stride", [(1, 0, 1), (255, 0, 257), (256, 0, 256), (250, 3, 255),
-                                            (254, 0, 260), (248, 8, 256), (5, 5, 9)])
+                                            (254, 0, 260), (248, 8, 256), (5, 5, 9),
+                                            (240, 0, 250)])
 def test_masked_copies_are_exact(dtype, offset, N, first, stride):
     rows, pad = 3, 300
     g = torch.Generator(device="cuda").manual_seed(2)
