@@ -134,7 +134,7 @@ def softmax(x, out=None, num_warps=None):
     M, N = x.shape
     out = torch.empty_like(x) if out is None else out
     BLOCK_N = newt.next_power_of_2(N)
-    rows = 0 if num_warps else rows_per_program(BLOCK_N, x.element_size())
+    rows = 0 if num_warps or BLOCK_N > 512 else rows_per_program(BLOCK_N, x.element_size())
     if rows:
         softmax_rows_kernel[(newt.cdiv(M, rows),)](x, out, M, N, x.stride(0), ROWS=rows,
                                                    BLOCK_N=BLOCK_N, num_warps=4)
@@ -194,7 +194,7 @@ def layernorm(x, w, b, eps=1e-5, out=None, num_warps=None):
     mean = torch.empty(M, device=x.device, dtype=torch.float32)
     rstd = torch.empty(M, device=x.device, dtype=torch.float32)
     BLOCK_N = newt.next_power_of_2(N)
-    rows = 0 if num_warps else rows_per_program(BLOCK_N, x.element_size())
+    rows = 0 if num_warps or BLOCK_N > 512 else rows_per_program(BLOCK_N, x.element_size())
     if rows:
         layernorm_rows_kernel[(newt.cdiv(M, rows),)](x, w, b, out, mean, rstd, M, N, x.stride(0),
                                                      eps, ROWS=rows, BLOCK_N=BLOCK_N, num_warps=4)
