@@ -257,10 +257,9 @@ MATMUL_CONFIGS = [
     newt.Config({"BLOCK_M": 64, "BLOCK_N": 128, "BLOCK_K": 64}, num_warps=4, num_stages=3),
     # 64x64 tiles give a 1024^3 problem 256 workgroups (one per CU)
     newt.Config({"BLOCK_M": 64, "BLOCK_N": 64, "BLOCK_K": 64}, num_warps=4, num_stages=4),
-    # 128-deep k-steps (128 KB of stages) halve the barriers: bf16 256x4096x4096
-    # 16.3 against 17.8 us for the tile above (x @ w.t(): 14.8 against 18.0),
-    # 1024x1024x4096 the same, 1024^3 7.0 either way
-    newt.Config({"BLOCK_M": 64, "BLOCK_N": 64, "BLOCK_K": 128}, num_warps=4, num_stages=4),
+    # (64x64x128 with 4 stages stays out of this list: with flushed caches, as
+    # the tuner times, it wins at 1024^3, where it then runs 7.0 us back to back
+    # against 6.0 for the tile above; it gained 9% at 256x4096x4096)
     # two waves per SIMD over a 64x128 tile: bf16 640x2048x2048 (320 such
     # tiles) 12.7 us against 15.1 for 64x64x64 and 15.5 for 128x128x64
     newt.Config({"BLOCK_M": 64, "BLOCK_N": 128, "BLOCK_K": 64}, num_warps=8, num_stages=4),
