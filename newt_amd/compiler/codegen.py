@@ -455,11 +455,10 @@ class Codegen(ast.NodeVisitor):
         return None
 
     def _meta_permute(self, meta, perm):
-        if meta[0] == "and":
-            parts = [self._meta_permute(m, perm) for m in meta[1]]
-            return None if any(m is None for m in parts) else ("and", parts)
-        if meta[0] == "cmp" and len(meta[2].shape) == len(perm):
+        if meta[0] == "cmp":
             return ("cmp", meta[1], self.permute(meta[2], perm))
+        if meta[0] == "and":
+            return ("and", [self._meta_permute(m, perm) for m in meta[1]])
         return None
 
     def permute(self, v, perm):
@@ -1470,7 +1469,7 @@ class Codegen(ast.NodeVisitor):
                 self.err(node, f"bitwise {sym} on floats")
             r = emit(wrap(lambda es: f"({es[0]} {sym} {es[1]})"))
             if sym == "&" and rd == tp.int1 and isinstance(r, Lazy):
-                r.meta = self._and_meta(a, b)
+                r.meta = self._and_meta(a, b, len(r.shape))
             return r
         if op == ast.Div:
             return emit(wrap(lambda es: f"({es[0]} / {es[1]})"))
@@ -1494,14 +1493,17 @@ class Codegen(ast.NodeVisitor):
             return emit(wrap(lambda es: f"{f}({es[0]}, {es[1]})"))
         self.err(node, f"unsupported operator {op.__name__}")
 
-    def _and_meta(self, a, b):
+    def _and_meta(self, a, b, rank):
+        """Comparisons of `a & b`, each at the result's rank: readers look its
+        extents and coefficients up by the result's dims (a lower-rank operand
+        broadcasts over the leading ones)."""
         parts = []
         for x in (a, b):
             m = getattr(x, "meta", None) if isinstance(x, Lazy) else None
             if m is None:
                 return None
             parts += m[1] if m[0] == "and" else [m]
-        return ("and", parts)
+        return ("and", [(kind, sym, self.expand_to_rank(diff, rank)) for kind, sym, diff in parts])
 
     def as_affine(self, v, rd):
         if isinstance(v, Affine):
