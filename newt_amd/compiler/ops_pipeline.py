@@ -913,7 +913,8 @@ class DotPipeline:
 
     def pipe_dma_condition(self, state):
         """Uniform condition under which every DMA tile of the slice just
-        visited is a whole in-bounds copy; consumes the slice's loads."""
+        visited is a whole in-bounds copy; consumes the slice's loads. Records
+        whether the branch-free loop writes a tile to LDS from registers."""
         if state["recs"] is None:
             self._init_recs(state)
         conds = []
@@ -921,6 +922,8 @@ class DotPipeline:
             X = self.locals.get(r["name"])
             if not isinstance(X, LazyLoad) or X.result is not None or tuple(X.shape) != r["shape"]:
                 self._no_pipe(state)
+            if state.get("ahead") or not r["dma"] or self.mask_all_true(X.mask, X.shape) is None:
+                state["reg_tiles"] = True
             if state.get("ahead"):
                 V = X if r["kdim"] == 1 else self.permute(X, (1, 0))
                 parts = None
@@ -981,7 +984,10 @@ class DotPipeline:
                           f"else newt::wait_vmcnt<0>();")
             else:
                 self.emit("newt::wait_vmcnt<0>();")
-            if fast and os.environ.get("NEWT_BARE_BARRIER", "0") == "1":
+            # the bare barrier publishes copies only: tiles written to LDS from
+            # registers need the fence's lgkmcnt(0) ahead of it
+            if (fast and os.environ.get("NEWT_BARE_BARRIER", "0") == "1"
+                    and not state.get("reg_tiles")):
                 self.emit("newt::barrier_nofence();")
             else:
                 self.emit("__syncthreads();")

@@ -805,8 +805,8 @@ __device__ __forceinline__ void join_k_groups(VT* acc, f32x4* buf, int tid) {
 // waits for all of this wave's LDS reads (lgkmcnt(0)) before the wave
 // arrives, including a fragment prefetch of a pipeline stage that the
 // barrier does not release. Callers wait for the copies the barrier publishes
-// (wait_vmcnt) first; reads of the stage the barrier releases have all been
-// consumed by then. The "memory" clobber keeps the compiler from moving
+// (wait_vmcnt) first and publish nothing that they wrote to LDS from registers;
+// reads of the stage the barrier releases have all been consumed by then. The "memory" clobber keeps the compiler from moving
 // memory accesses across it.
 __device__ __forceinline__ void barrier_nofence() { asm volatile("s_barrier" ::: "memory"); }
 

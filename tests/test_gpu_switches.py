@@ -75,6 +75,27 @@ def test_switch_keeps_results(monkeypatch, var, value):
     assert torch.equal(W.add(xa, ya), xa + ya)
 
 
+@pytest.mark.parametrize("cfg", [(64, 64, 64, 8, 3), (64, 64, 64, 4, 2), (128, 128, 32, 4, 4)])
+@pytest.mark.parametrize("var,value", [("NEWT_BARE_BARRIER", "1"), ("NEWT_BUFFER_DMA", "0"),
+                                       ("NEWT_PIPE_CLAMP", "0"), ("NEWT_VEC", "2")])
+def test_switch_keeps_odd_strided_products(monkeypatch, var, value, cfg):
+    """Tiles written to LDS from registers (odd row strides, one operand with
+    no unit stride)."""
+    from newt_amd import workloads as W
+    monkeypatch.setenv(var, value)
+    BM, BN, BK, nw, ns = cfg
+    print(f"{var}={value} odd strides, tile {cfg}", flush=True)
+    M, N, K = 300, 265, 777
+    a = seeded((M, K), 70, scale=K ** -0.5, dtype=torch.float16)
+    b = seeded((K, N), 71, scale=K ** -0.5, dtype=torch.float16)
+    ref = orc.matmul(npf(a), npf(b), "float16")
+    for x in (a, torch.stack((a, a), dim=2)[:, :, 0]):
+        c = W.matmul(x, b, config=newt.Config({"BLOCK_M": BM, "BLOCK_N": BN, "BLOCK_K": BK},
+                                              num_warps=nw, num_stages=ns))
+        assert orc.rel_frobenius(npf(c), ref) <= 1e-2, x.stride()
+        assert orc.ulp_violations(npf(c), ref, "float16") == 0, x.stride()
+
+
 @pytest.mark.parametrize("B,H,S", [(2, 4, 1000), (1, 3, 700), (1, 16, 513)])
 def test_heaviest_first_order_is_bit_identical(monkeypatch, B, H, S):
     """The causal examples/05 form runs heaviest first (its key loop grows with
