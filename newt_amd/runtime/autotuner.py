@@ -24,6 +24,7 @@ is a single merge of the call's keyword arguments with the chosen Config.
 """
 
 import functools
+import inspect
 
 
 class Config:
@@ -75,9 +76,12 @@ class _Binding:
     def tuning_key(self, key_names):
         import torch
 
-        def part(v):
+        def part(name):
+            if callable(name):
+                return name(*[self.values[n] for n in inspect.signature(name).parameters])
+            v = self.values.get(name)
             return tuple(v.shape) if hasattr(v, "shape") else v
-        head = tuple(part(self.values.get(name)) for name in key_names)
+        head = tuple(part(name) for name in key_names)
         dtypes = tuple(str(v.dtype) for v in self.values.values() if isinstance(v, torch.Tensor))
         return head + dtypes
 
@@ -168,14 +172,22 @@ class Autotuner:
         import torch
 
         names = self.param_names[:len(args)]
-        if len(names) != len(args) or not set(self.key) <= set(names):
+        if len(names) != len(args):
             return None
-        parts = []
+        parts, rules = [], {}
         for name in self.key:
-            i = names.index(name)
-            parts.append(f"a[{i}].shape" if hasattr(args[i], "shape") else f"a[{i}]")
+            reads = list(inspect.signature(name).parameters) if callable(name) else [name]
+            if not set(reads) <= set(names):
+                return None
+            if callable(name):
+                rule = f"r{len(rules)}"
+                rules[rule] = name
+                parts.append(f"{rule}({', '.join(f'a[{names.index(n)}]' for n in reads)})")
+            else:
+                i = names.index(name)
+                parts.append(f"a[{i}].shape" if hasattr(args[i], "shape") else f"a[{i}]")
         parts += [f"a[{i}].dtype" for i, v in enumerate(args) if isinstance(v, torch.Tensor)]
-        return eval(f"lambda a: ({''.join(p + ', ' for p in parts)})")
+        return eval(f"lambda a: ({''.join(p + ', ' for p in parts)})", rules)
 
     def _launch(self, grid, *args, **kwargs):
         # a positional call whose key was tuned before: one generated expression
@@ -215,7 +227,10 @@ class Autotuner:
 
 
 def autotune(configs, key, reset_to_zero=None):
-    """@newt.autotune(configs, key, reset_to_zero=None) over a @newt.jit kernel."""
+    """@newt.autotune(configs, key, reset_to_zero=None) over a @newt.jit kernel.
+    key: names of arguments whose values (shapes of tensors) select the tuned
+    Config; an entry may also be a function of arguments, which it takes by
+    its own parameters' names, for a class of values that share one Config."""
     return lambda jitfn: Autotuner(jitfn, configs, key, reset_to_zero)
 
 

@@ -236,6 +236,22 @@ def matmul_kernel(a_ptr, b_ptr, c_ptr, M, N, K,
     nl.store(c_ptrs, acc.to(c_ptr.dtype.element_ty), mask=c_mask)
 
 
+def operand_layout(sam, sak, sbk, sbn):
+    """What of the operands' strides decides which tiles serve them, as a part
+    of the tuning key: which dim has unit stride and whether the other keeps
+    16-byte rows. One shape in two layouts (x @ w.t() and then dy @ w of a
+    square weight, or an odd row stride) has different best tiles: the best of
+    bf16 x[16,4096] @ w.t(), 16x16x512 at 6.7 us, takes 18.5 on w itself, where
+    16x32x128 takes 11.4; of fp32 512^3, 32x32x64 at 5.9, takes 17.3, where
+    32x64x32 takes 7.3."""
+    # per stride: 1, a multiple of 8 elements (0) or any other (2)
+    return (sam if sam == 1 else sam % 8 and 2, sak if sak == 1 else sak % 8 and 2,
+            sbk if sbk == 1 else sbk % 8 and 2, sbn if sbn == 1 else sbn % 8 and 2)
+
+
+MATMUL_KEY = ["M", "N", "K", operand_layout]
+
+
 # gfx950 search space: 64-wide waves, 160 KB LDS per CU, 256 CUs. The k-loop is
 # software-pipelined num_stages deep through distinct LDS stages, so tiles of
 # 256x256 with BLOCK_K=32 and 4 stages (128 KB) give each CU one workgroup:
@@ -270,7 +286,7 @@ MATMUL_CONFIGS = [
     newt.Config({"BLOCK_M": 64, "BLOCK_N": 64, "BLOCK_K": 64}, num_warps=8, num_stages=3),
 ]
 
-matmul_tuned = newt.autotune(configs=MATMUL_CONFIGS, key=["M", "N", "K"])(matmul_kernel)
+matmul_tuned = newt.autotune(configs=MATMUL_CONFIGS, key=MATMUL_KEY)(matmul_kernel)
 
 # Products whose 64x64 tiles do not fill the 256 CUs (few rows, few columns or
 # small all round) are bound by the bytes that the launch keeps in flight, not
@@ -299,8 +315,7 @@ MATMUL_CONFIGS_SMALL = [
     newt.Config({"BLOCK_M": 64, "BLOCK_N": 32, "BLOCK_K": 64}, num_warps=4, num_stages=4),
     newt.Config({"BLOCK_M": 64, "BLOCK_N": 64, "BLOCK_K": 64}, num_warps=8, num_stages=3),
 ]
-matmul_tuned_small = newt.autotune(configs=MATMUL_CONFIGS_SMALL,
-                                   key=["M", "N", "K"])(matmul_kernel)
+matmul_tuned_small = newt.autotune(configs=MATMUL_CONFIGS_SMALL, key=MATMUL_KEY)(matmul_kernel)
 
 # fp32 operands run on the fp32 MFMA (v_mfma_f32_32x32x2_f32, full precision;
 # gfx950 has no tf32) through the same pipelined k-loop: 16-deep k-steps keep
@@ -313,7 +328,7 @@ MATMUL_CONFIGS_FP32 = [
     # two waves per SIMD: 2048^3 118.4 against 119.9 us for the tile above
     newt.Config({"BLOCK_M": 128, "BLOCK_N": 128, "BLOCK_K": 32}, num_warps=8, num_stages=3),
 ]
-matmul_tuned_fp32 = newt.autotune(configs=MATMUL_CONFIGS_FP32, key=["M", "N", "K"])(matmul_kernel)
+matmul_tuned_fp32 = newt.autotune(configs=MATMUL_CONFIGS_FP32, key=MATMUL_KEY)(matmul_kernel)
 
 # fp32 products whose 128x128 tiles do not fill the 256 CUs: the fp32 MFMA is
 # slow enough (64 cycles for 32x32x2) that a launch takes as long as its
@@ -332,7 +347,7 @@ MATMUL_CONFIGS_FP32_SMALL = [
     newt.Config({"BLOCK_M": 128, "BLOCK_N": 128, "BLOCK_K": 32}, num_warps=8, num_stages=3),
 ]
 matmul_tuned_fp32_small = newt.autotune(configs=MATMUL_CONFIGS_FP32_SMALL,
-                                        key=["M", "N", "K"])(matmul_kernel)
+                                        key=MATMUL_KEY)(matmul_kernel)
 
 
 def matmul(a, b, c=None, config=None):
@@ -340,8 +355,7 @@ def matmul(a, b, c=None, config=None):
     K2, N = b.shape
     assert K == K2
     c = torch.empty(M, N, device=a.device, dtype=a.dtype) if c is None else c
-    args = (a, b, c, M, N, K, a.stride(0), a.stride(1), b.stride(0), b.stride(1),
-            c.stride(0), c.stride(1))
+    args = (a, b, c, M, N, K, *a.stride(), *b.stride(), *c.stride())
     if config is None:
         grid = lambda meta: (newt.cdiv(M, meta["BLOCK_M"]), newt.cdiv(N, meta["BLOCK_N"]))
         if a.dtype == torch.float32:
