@@ -585,6 +585,16 @@ def attention_tile(S, heads, D, causal):
       29.7 / 36.6 / 31.8, [112, 1024] 52.9 / 57.5 / 49.7 / 52.0, [40, 2048] 58.7 /
       62.4 / 52.2 / 59.8, [64, 2048] 76.1 / 87.4 / 80.0 / 90.0, [80, 2048] 104 / 114 /
       96 / 112, [128, 2048] 166 / 188 / 168 / 192;
+      heads that the 8 XCDs share evenly, S from 2048 (256x8 / 128x4): [40, 2048]
+      63.9 / 56.5, [40, 2304] 65.6 / 67.2, [48, 2048] 64.9 / 65.7, [40, 2560] 77.3 /
+      80.7, [32, 3584] 104 / 111, [56, 2048] 75.7 / 73.4, [40, 3072] 102 / 103,
+      [64, 2048] 76.9 / 80.4, [32, 4096] 131 / 138, [16, 8192] 235 / 252, [72, 2048]
+      97 / 88, [48, 3072] 129 / 119, [128, 2048] 156 / 155, [64, 4096] 275 / 267,
+      [128, 4096] 547 / 547, [32, 8192] 475 / 490: from 352 programs to the second
+      full round, and from four rounds on;
+      other heads: [47, 2048] 89 / 83, [49, 2048] 108 / 89, [63, 2048] 111 / 101,
+      [65, 2048] 119 / 108, [31, 4096] 185 / 170, [33, 4096] 196 / 176, [129, 2048]
+      206 / 180, [125, 4096] 604 / 558, [65, 8192] 1080 / 1047;
       causal, D 64: [64, 1024] 24.3 / 24.2 / 23.6 / 20.2, [256, 1024] 74.2 / 64.2 /
       60.7 / 58.7, [64, 2048] 52.1 / 53.9 / 50.0 / 55.9, [32, 2048] 41.9 / 32.6 /
       30.1 / 28.3."""
@@ -605,8 +615,11 @@ def attention_tile(S, heads, D, causal):
         return (64, 4) if S <= 1024 or rounds(128) < 4 else (128, 4)
     if programs <= 256:
         return (128, 8) if programs > 160 and S > 512 else (64, 4)
-    # long sequences: one and a half, two, and from four rounds on 256 rows win
-    if S >= 2048 and (programs >= 1024 or programs in (384, 512)):
+    # long sequences whose heads divide over the 8 XCDs: a round of long programs
+    # pairs with one of short ones up to two rounds, and from four rounds on they
+    # balance by their number; in between, and where an XCD holds a part of a
+    # head, the halves on 4 waves fill the last round better
+    if S >= 2048 and heads % 8 == 0 and (programs >= 1024 or 352 < programs <= 512):
         return 256, 8
     return 128, 4
 
