@@ -754,7 +754,12 @@ class DotPipeline:
     def _join_ksplit(self, state, mark):
         """Around a loop whose waves split k: every group but the first starts
         from zero, and afterwards each group adds all shares, in group order
-        (so every wave holds the same sums), through the stages' LDS.
+        (so every wave holds the same sums), through the first stage's LDS, in
+        as many parts as it takes: with an area of its own, the join set the
+        LDS of the whole kernel (fp16 64x64x64 on 8 waves with 3 stages 80 KB
+        instead of 48, fp32 64x64x32 on 8 with 4 96 instead of 64, a workgroup
+        per CU less each; fp32 1500x700x1003 43.7 -> 38.2 us on the latter,
+        level where a launch has one workgroup per CU).
 
         This is for output tiles too small to give every wave rows or columns
         of its own (16x16 to 64x64 per workgroup, a product with few rows):
@@ -770,14 +775,17 @@ class DotPipeline:
         zero = "f32x16" if acc.vec == 16 else "f32x4"
         self._insert_lines(mark, [f"if ({group}) {{"]
                            + [f"  {acc.var}[{i}] = ({zero})(0.0f);" for i in range(nv)] + ["}"])
-        nbytes = 4 * self.T * L.nslots
+        quads = L.nslots // 4
         area, size = self.lds_arrays[state["lds_idx"][0]]
-        if nbytes > size:
-            area = f"(_lds + {self.lds_arena(nbytes)})"
+        if size < 16 * self.T:      # 16 waves on a stage of shallow k-steps
+            size = 16 * self.T
+            area = f"(_lds + {self.lds_arena(size)})"
+        parts = -(-quads // (size // (16 * self.T)))
+        part = -(-quads // parts)
         # every wave's copies have landed and every wave is done with the stages
         self.emit("newt::wait_vmcnt<0>();")
         self.emit("__syncthreads();")
-        self.emit(f"newt::join_k_groups<{acc.vec}, {nv}, {rep}, {lanes}>({acc.var}, "
+        self.emit(f"newt::join_k_groups<{acc.vec}, {nv}, {rep}, {lanes}, {part}>({acc.var}, "
                   f"(f32x4*){area}, _tid);")
         self.emit("__syncthreads();")
 

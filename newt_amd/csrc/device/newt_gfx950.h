@@ -776,29 +776,31 @@ __device__ __forceinline__ void wait_vmcnt() {
 // Sums of REP groups of LANES threads that each hold a share of the same
 // tile: thread t of every group holds NV vectors of V floats of the same
 // elements. Every group gets the sum of all shares, taken in group order, so
-// all groups hold the same bits. buf: REP * LANES * NV * V floats of LDS,
-// written with 16-byte accesses by consecutive lanes.
-template <int V, int NV, int REP, int LANES, typename VT>
+// all groups hold the same bits. Quads of floats go through buf QC at a time:
+// REP * LANES * QC of them, written with 16-byte accesses by consecutive lanes.
+template <int V, int NV, int REP, int LANES, int QC, typename VT>
 __device__ __forceinline__ void join_k_groups(VT* acc, f32x4* buf, int tid) {
   const int g = tid / LANES, t = tid % LANES;
   constexpr int Q = V / 4;
 #pragma unroll
-  for (int i = 0; i < NV; ++i)
+  for (int c = 0; c < NV * Q; c += QC) {
+    if (c) __syncthreads();
 #pragma unroll
-    for (int q = 0; q < Q; ++q)
-      buf[((i * Q + q) * REP + g) * LANES + t] =
-          f32x4{acc[i][4 * q], acc[i][4 * q + 1], acc[i][4 * q + 2], acc[i][4 * q + 3]};
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < NV; ++i)
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      f32x4 s = buf[(i * Q + q) * REP * LANES + t];
-#pragma unroll
-      for (int r = 1; r < REP; ++r) s += buf[((i * Q + q) * REP + r) * LANES + t];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[i][4 * q + e] = s[e];
+    for (int j = c; j < c + QC && j < NV * Q; ++j) {
+      const VT& v = acc[j / Q];
+      const int e = 4 * (j % Q);
+      buf[((j - c) * REP + g) * LANES + t] = f32x4{v[e], v[e + 1], v[e + 2], v[e + 3]};
     }
+    __syncthreads();
+#pragma unroll
+    for (int j = c; j < c + QC && j < NV * Q; ++j) {
+      f32x4 s = buf[(j - c) * REP * LANES + t];
+#pragma unroll
+      for (int r = 1; r < REP; ++r) s += buf[((j - c) * REP + r) * LANES + t];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[j / Q][4 * (j % Q) + e] = s[e];
+    }
+  }
 }
 
 // Workgroup barrier without the fence __syncthreads() carries. That fence

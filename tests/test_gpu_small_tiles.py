@@ -56,6 +56,16 @@ def test_waves_split_k_fp32(M, N, K, ta, tb, cfg):
     check(M, N, K, ta, tb, torch.float32, cfg)
 
 
+@pytest.mark.parametrize("dtype,cfg", [
+    (torch.float16, (64, 64, 64, 8, 3)), (torch.bfloat16, (64, 128, 32, 16, 3)),
+    (torch.bfloat16, (64, 128, 64, 16, 2)), (torch.float32, (32, 64, 64, 8, 4)),
+    (torch.float32, (64, 64, 32, 8, 4)), (torch.float32, (32, 64, 32, 4, 2))])
+@pytest.mark.parametrize("M,N,K", [(128, 128, 512), (70, 131, 1033)])
+def test_shares_joined_in_parts(M, N, K, dtype, cfg):
+    """Shares of more than one stage's LDS, and of less than one part each."""
+    check(M, N, K, False, False, dtype, cfg)
+
+
 @pytest.mark.parametrize("M,N,K", [(16, 1024, 1024), (1, 512, 768), (100, 1000, 520),
                                    (960, 1024, 128)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
