@@ -53,6 +53,10 @@ _ELT_FOOTPRINT = 1 << 15
 # gfx950 tilings dot kernels start from: (grid tile, inner tile, waves, stages)
 _DOT_SEEDS = ((256, 32, 4, 4), (256, 32, 8, 4), (128, 64, 4, 3), (128, 32, 4, 4))
 
+# exact shapes whose tuning keys a kernel keeps ready (the keys themselves are
+# by power-of-two class: varying lengths must not grow a kernel for good)
+_MAX_KEYS = 1024
+
 
 def _pow2_at_least(n):
     n = int(n)
@@ -408,7 +412,7 @@ class Kernel:
         self.trials = []        # the latest tuning's (Config, ms or None, note)
         self._specs = {}        # argument signature -> _Specialization
         self._chosen = {}       # tuning key -> Config
-        self._keys = {}         # (specialisation, shapes) -> tuning key
+        self._keys = {}         # (specialisation, shapes) -> tuning key, at most _MAX_KEYS
         self._last = None
 
     # ---- public API
@@ -464,6 +468,8 @@ class Kernel:
         quick = (spec, tuple([a.shape for a in args if isinstance(a, torch.Tensor)]))
         key = self._keys.get(quick)
         if key is None:
+            if len(self._keys) >= _MAX_KEYS:
+                self._keys.clear()
             key = self._keys[quick] = self.tuning_key(spec, args)
         cfg = self._chosen.get(key)
         if cfg is None:

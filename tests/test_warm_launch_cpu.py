@@ -114,3 +114,24 @@ def test_deuteron_launch_arguments():
         assert len(args) == len(want)
         assert all(p is q or p == q for p, q in zip(args, want))
         assert kw["num_warps"] == 2 and kw["BLOCK_TILE_M"] == 8 and 64 in kw.values()
+
+
+@dt.kernel(autotune=False)
+def doubled(x, out):
+    for t in dt.tile(x.shape[0]):
+        out[t] = x[t] * 2.0
+
+
+def test_varying_lengths_keep_a_bounded_table():
+    """One length after another: the classes' configurations stay, the table
+    of exact shapes does not grow for the life of the kernel."""
+    from newt_amd.deuteron import runtime
+    spec, classes = None, {}
+    x = torch.zeros(5000)
+    for n in (*range(1, 5000), 3, 4999):
+        a = (x[:n], x[:n])
+        spec = doubled._specialize(a)
+        cfg = doubled._choose(spec, a)
+        assert classes.setdefault(doubled.tuning_key(spec, a), cfg) is cfg
+        assert len(doubled._keys) <= runtime._MAX_KEYS
+    assert len(doubled._chosen) == len(classes) == 14
