@@ -184,8 +184,8 @@ static PyObject* py_run(PyObject* self, PyObject* const* a, Py_ssize_t na) {
   Py_ssize_t nargs = PyTuple_GET_SIZE(args), ncx = PyTuple_GET_SIZE(cx);
   if (nargs > MAX_ARGS) Py_RETURN_FALSE;
 
-  /* the launch grid: an int or a tuple of 1-3 ints (a callable grid takes the
-     Python path) */
+  /* the launch grid: an int or a tuple of 1-3 ints (the caller has evaluated a
+     callable one); any other form takes the Python path */
   long g[3] = {1, 1, 1};
   if (PyLong_CheckExact(grid)) {
     g[0] = PyLong_AsLong(grid);

@@ -442,12 +442,16 @@ class JITFunction:
             except (RuntimeError, AssertionError):
                 pass                # no GPU: the Python path reports what is wrong
         if C and _Dev.ready and launch_events is None:
-            if callable(grid):
-                grid = self._grid_of(grid, args, kwargs)
             try:
-                r = C.run(self._ctable, self._cx_pos, grid, args, kwargs)
-            except TypeError:     # an unhashable constexpr: the Python path reports it
-                r = False
+                if callable(grid):
+                    grid = self._grid_of(grid, args, kwargs)
+            except Exception:
+                r = False       # the Python path checks the arguments before it asks the grid
+            else:
+                try:
+                    r = C.run(self._ctable, self._cx_pos, grid, args, kwargs)
+                except TypeError:     # an unhashable constexpr: the Python path reports it
+                    r = False
             if r is None:
                 return
             if type(r) is int:

@@ -2,6 +2,8 @@
 with stand-in kernels: the short path passes what the first launch passes and
 gives way to the full one whenever a fact it rests on changes."""
 
+import re
+
 import pytest
 import torch
 
@@ -135,3 +137,26 @@ def test_varying_lengths_keep_a_bounded_table():
         assert classes.setdefault(doubled.tuning_key(spec, a), cfg) is cfg
         assert len(doubled._keys) <= runtime._MAX_KEYS
     assert len(doubled._chosen) == len(classes) == 14
+
+
+@pytest.mark.parametrize("args,kw,error", [
+    ((1,), {}, "missing kernel arguments: ['n']"), ((), {"n": 1}, "missing kernel arguments: ['x_ptr']"),
+    ((1, 2, 3, 4), {}, "takes 3 arguments but 4 were given"),
+    ((1, 2), {"BLOK": 64}, "unknown kernel arguments: ['BLOK']")])
+def test_wrong_arguments_are_named_before_the_grid_reads_them(monkeypatch, args, kw, error):
+    from newt_amd.runtime import jit as J
+    monkeypatch.setattr(J, "_C_LAUNCH", type("C", (), {"run": staticmethod(lambda *a: False)}))
+    monkeypatch.setattr(J._Dev, "ready", True)
+    monkeypatch.setattr(J._Dev, "device", staticmethod(lambda: 0))
+    with pytest.raises(TypeError, match=re.escape(error)):
+        k[lambda m: (m["n"] // m["BLOK"] if "BLOK" in m else m["x_ptr"] + m["n"],)](*args, **kw)
+
+
+def test_a_grids_own_error_reaches_the_caller(monkeypatch):
+    from newt_amd.runtime import jit as J
+    monkeypatch.setattr(J, "_C_LAUNCH", type("C", (), {"run": staticmethod(lambda *a: False)}))
+    monkeypatch.setattr(J._Dev, "ready", True)
+    monkeypatch.setattr(J._Dev, "device", staticmethod(lambda: 0))
+    monkeypatch.setattr(J.JITFunction, "_slow_path", lambda *a: (None, None))
+    with pytest.raises(KeyError, match="ROWS"):
+        k[lambda m: (m["ROWS"],)](1, 640)
