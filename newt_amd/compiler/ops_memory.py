@@ -20,12 +20,13 @@ whose 16-byte alignment is not proven (rows of an odd stride) is accessed
 with the same vector instructions at its element's alignment.
 """
 
+import math
 import os
 
 from . import layouts as lo
 from . import types as tp
 from .codegen import CompileError
-from .values import Affine, Block, Const, Lazy, LazyLoad, PtrBlock, Reg, Scalar, Sym
+from .values import Affine, Block, Const, Fill, Lazy, LazyLoad, PtrBlock, Reg, Scalar, Sym
 
 
 class MemoryOps:
@@ -192,6 +193,15 @@ class MemoryOps:
                 return None
         return meta[1]
 
+    @staticmethod
+    def zero_fill(other):
+        """Whether a masked load's `other` is the zero that a buffer load out
+        of range returns (all bits clear: not -0.0)."""
+        if isinstance(other, Fill):
+            other = other.value
+        return other is None or (isinstance(other, Const) and other.pyval == 0
+                                 and math.copysign(1.0, other.pyval) > 0)
+
     def run_mask(self, mask, L, chunk):
         """How `mask` runs over the aligned runs of `chunk` slots along the
         contiguous dim of L: 'uniform' (one value per run), 'prefix' (true up
@@ -275,7 +285,7 @@ class MemoryOps:
                             for a, c in off.coefs.items())
                     and esz * sum(c.const * (off.shape[a] - 1) for a, c in off.coefs.items()
                                   if off.shape[a] > 1) < (1 << 31) - 16)
-        zero_fill = other is None or (isinstance(other, Const) and other.pyval == 0)
+        zero_fill = self.zero_fill(other)
         rd = (lambda e: f"__builtin_nontemporal_load(&{e})") if nt else (lambda e: e)
 
         def oth(s):

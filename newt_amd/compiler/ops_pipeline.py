@@ -59,7 +59,7 @@ import os
 
 from . import layouts as lo
 from . import types as tp
-from .values import Affine, Block, Const, Fill, Lazy, LazyLoad, Reg, Scalar, Staged, Sym
+from .values import Affine, Block, Const, Lazy, LazyLoad, Reg, Scalar, Staged, Sym
 
 _SIDE_EFFECTS = {"store", "atomic_add", "atomic_max", "atomic_min"}
 
@@ -615,8 +615,7 @@ class DotPipeline:
         if V.mask is None:
             return True
         meta = getattr(V.mask, "meta", None) if isinstance(V.mask, Lazy) else None
-        other = X.other.value if isinstance(X.other, Fill) else X.other
-        if not meta or not (other is None or (isinstance(other, Const) and other.pyval == 0)):
+        if not meta or not self.zero_fill(X.other):
             return False
         call = plan["flat"][plan["staged"][r["name"]]["index"]].value
         masks = [k.value for k in call.keywords if k.arg == "mask"] + list(call.args[1:2])
@@ -1099,10 +1098,7 @@ class DotPipeline:
         mask's comparisons that no iteration changes). The copy drops a masked
         16-byte chunk by an offset past the buffer's end, which writes zeros,
         so the mask must be uniform over chunks and `other` zero."""
-        other = X.other
-        if isinstance(other, Fill):
-            other = other.value
-        if not (other is None or (isinstance(other, Const) and other.pyval == 0)):
+        if not self.zero_fill(X.other):
             return False, ()
         parts = self.chunk_mask(V.mask, 1 if fmt == "k" else 0, 16 // dt.itemsize)
         if parts is None or os.environ.get("NEWT_BUFFER_DMA", "1") == "0":

@@ -1032,3 +1032,18 @@ def test_whole_body_versioning_leaves_runtime_ifs_alone():
     src = compile_source(km, args, {"BLOCK": 256})[0]
     assert src.count("if ((true)) {") == 2 and src.count("(n > 8)") == 2
     isa(src)
+
+
+@pytest.mark.parametrize("other,filled", [(0.0, False), (0, False), (-0.0, True), (1.5, True)])
+def test_masked_runs_read_out_of_range_only_for_a_positive_zero(other, filled):
+    """A 16-byte run whose mask is uniform is loaded out of a buffer's range,
+    which gives +0.0: any other fill, -0.0 among them, is written after it."""
+    def k(x_ptr, o_ptr, N, stride, OTHER: nl.constexpr, BLOCK: nl.constexpr):
+        row, cols = nl.program_id(0), nl.arange(0, BLOCK)
+        x = nl.load(x_ptr + row * stride + cols, mask=cols < N, other=OTHER)
+        nl.store(o_ptr + row * BLOCK + cols, x)
+
+    src, _ = compile_source(k, {"x_ptr": (F32P, A16), "o_ptr": (F32P, A16), "N": (tp.int32, D16),
+                                "stride": (tp.int32, D16)}, {"OTHER": other, "BLOCK": 1024})
+    assert "newt::buf_load_vec<float, 4>" in src
+    assert bool(re.search(r"if \(!\(.*\)\) \{\n\s+_r\d+\[0\] = ", src)) == filled

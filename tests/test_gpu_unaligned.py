@@ -77,3 +77,28 @@ def test_row_kernels_on_odd_rows(M, N, offset):
     # fp32 error of its terms
     bound = 2.0 ** -11 * ref.abs() + 2.0 ** -24 + 1e-5 * (ref - b.double()).abs() + 1e-6 * b.abs()
     assert bool(((out.double() - ref).abs() <= bound).all())
+
+
+@newt.jit
+def padded_rows_k(x_ptr, o_ptr, N, stride, NEGATIVE: nl.constexpr, OTHER: nl.constexpr,
+                  BLOCK: nl.constexpr):
+    row = nl.program_id(0)
+    cols = nl.arange(0, BLOCK)
+    if NEGATIVE:
+        v = nl.load(x_ptr + row * stride + cols, mask=cols < N, other=-0.0)
+    else:
+        v = nl.load(x_ptr + row * stride + cols, mask=cols < N, other=OTHER)
+    nl.store(o_ptr + row * BLOCK + cols, v)
+
+
+@pytest.mark.parametrize("other", [0.0, -0.0, 2.5, float("-inf")])
+@pytest.mark.parametrize("N", [16, 240, 250, 256])
+def test_fill_value_keeps_its_bits(N, other):
+    g = torch.Generator(device="cuda").manual_seed(4)
+    x = torch.randn(3, 272, generator=g, device="cuda")
+    o = torch.full((3, 256), float("nan"), device="cuda")
+    padded_rows_k[(3,)](x, o, N, 272, NEGATIVE=str(other) == "-0.0", OTHER=other, BLOCK=256,
+                        num_warps=1)
+    want = torch.full((3, 256), other, device="cuda")
+    want[:, :N] = x[:, :N]
+    assert torch.equal(o.view(torch.int32), want.view(torch.int32))
