@@ -24,7 +24,7 @@ the K and V tiles of flash attention):
     ran 2-4x slower than a whole tile and the launch waited for it: fp16
     1000x1024x776 14.5 -> 6.8 us on 64x64x64 tiles, 1319x1600x1280 32.5 ->
     13.8, 777x1000x1032 26.6 -> 8.3, 4100x4104x4096 296 -> 157; causal
-    attention [4,32,4096,128], whose register tail spilled, 570 -> 555);
+    attention [4,32,4096,128], whose register tail spilled, 562 -> 551);
     other tiles (strided operands, masks or bounds inside a chunk) take a
     register path with the masked loads' `other` fill, written with ds_write
     and hinted cold;

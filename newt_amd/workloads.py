@@ -273,7 +273,10 @@ MATMUL_CONFIGS = [
     newt.Config({"BLOCK_M": 64, "BLOCK_N": 128, "BLOCK_K": 64}, num_warps=4, num_stages=3),
     # 64x64 tiles give a 1024^3 problem 256 workgroups (one per CU)
     newt.Config({"BLOCK_M": 64, "BLOCK_N": 64, "BLOCK_K": 64}, num_warps=4, num_stages=4),
-    # (64x64x128 with 4 stages stays out of this list: with flushed caches, as
+    # (64x64x64 on 4 waves with 3 stages left this list: of eight products from
+    # 1024x1024x256 to 256x4096x4096 in four layouts each it was ahead of the
+    # others in one, odd rows of the latter, 25.3 against 26.1 us.
+    # 64x64x128 with 4 stages stays out: with flushed caches, as
     # the tuner times, it wins at 1024^3, where it then runs 7.0 us back to back
     # against 6.0 for the tile above; it gained 9% at 256x4096x4096)
     # two waves per SIMD over a 64x128 tile: bf16 640x2048x2048 (320 such
@@ -333,9 +336,9 @@ matmul_tuned_fp32 = newt.autotune(configs=MATMUL_CONFIGS_FP32, key=MATMUL_KEY)(m
 # fp32 products whose 128x128 tiles do not fill the 256 CUs: the fp32 MFMA is
 # slow enough (64 cycles for 32x32x2) that a launch takes as long as its
 # busiest CU has MFMAs, so the tile is what divides the work most evenly.
-# 1024^3 (64 tiles of 128x128) 61.6 -> 21.3 us on 64x64x32, of 13.7 us of MFMA
-# work per CU; 512^3 7.1, x @ w.t() 5.5; [16,4096] @ [4096,4096] 33.1, x @ w.t()
-# 18.9 (67 MB; 32x32 tiles serve a transposed w only); 1500x700x1003 38.9.
+# 1024^3 (64 tiles of 128x128) 61.7 -> 18.6 us on 64x64x32, of 13.7 us of MFMA
+# work per CU; 512^3 7.3, x @ w.t() 5.9; [16,4096] @ [4096,4096] 33.2, x @ w.t()
+# 19.5 (67 MB; 32x32 tiles serve a transposed w only); 1500x700x1003 33.3.
 # From 256 tiles of 128x128 on (2048^3) the larger list is level or ahead.
 MATMUL_CONFIGS_FP32_SMALL = [
     newt.Config({"BLOCK_M": 32, "BLOCK_N": 32, "BLOCK_K": 64}, num_warps=4, num_stages=4),
