@@ -588,13 +588,15 @@ def attention_tile(S, heads, D, causal):
       29.7 / 36.6 / 31.8, [112, 1024] 52.9 / 57.5 / 49.7 / 52.0, [40, 2048] 58.7 /
       62.4 / 52.2 / 59.8, [64, 2048] 76.1 / 87.4 / 80.0 / 90.0, [80, 2048] 104 / 114 /
       96 / 112, [128, 2048] 166 / 188 / 168 / 192;
-      heads that the 8 XCDs share evenly, S from 2048 (256x8 / 128x4): [40, 2048]
-      63.9 / 56.5, [40, 2304] 65.6 / 67.2, [48, 2048] 64.9 / 65.7, [40, 2560] 77.3 /
-      80.7, [32, 3584] 104 / 111, [56, 2048] 75.7 / 73.4, [40, 3072] 102 / 103,
-      [64, 2048] 76.9 / 80.4, [32, 4096] 131 / 138, [16, 8192] 235 / 252, [72, 2048]
-      97 / 88, [48, 3072] 129 / 119, [128, 2048] 156 / 155, [64, 4096] 275 / 267,
-      [128, 4096] 547 / 547, [32, 8192] 475 / 490: from 352 programs to the second
-      full round, and from four rounds on;
+      heads that the 8 XCDs share evenly, S from 2048 (256x8 / 128x4), up to two
+      rounds: [32, 2816] 75.5 / 71.1, [16, 5888] 144 / 133, [16, 6144] 150 / 147,
+      [24, 4096] 104 / 106, [40, 2560] 75.8 / 79.3, [32, 3328] 89.0 / 96.5, [24, 4608]
+      122 / 132, [16, 7168] 178 / 198, [40, 3072] 98.6 / 102, [48, 2560] 87.6 / 87.8,
+      [64, 2048] 75.4 / 79.6, [16, 8192] 228 / 245, [40, 3328] 121 / 113, [24, 5632] 179 /
+      177; with an odd number of heads per XCD in 8 or 9 blocks [56, 2048] 75.2 /
+      72.7, [56, 2304] 87.8 / 83.3, [40, 2304] 64.3 / 65.9; from four rounds on
+      [128, 2048] 156 / 155, [64, 4096] 275 / 267, [128, 4096] 547 / 547, [32, 8192] 475 /
+      490;
       other heads: [47, 2048] 89 / 83, [49, 2048] 108 / 89, [63, 2048] 111 / 101,
       [65, 2048] 119 / 108, [31, 4096] 185 / 170, [33, 4096] 196 / 176, [129, 2048]
       206 / 180, [125, 4096] 604 / 558, [65, 8192] 1080 / 1047;
@@ -618,11 +620,14 @@ def attention_tile(S, heads, D, causal):
         return (64, 4) if S <= 1024 or rounds(128) < 4 else (128, 4)
     if programs <= 256:
         return (128, 8) if programs > 160 and S > 512 else (64, 4)
-    # long sequences whose heads divide over the 8 XCDs: a round of long programs
-    # pairs with one of short ones up to two rounds, and from four rounds on they
-    # balance by their number; in between, and where an XCD holds a part of a
-    # head, the halves on 4 waves fill the last round better
-    if S >= 2048 and heads % 8 == 0 and (programs >= 1024 or 352 < programs <= 512):
+    # long sequences whose heads divide over the 8 XCDs: a launch of up to two
+    # rounds lasts as long as its longest program, which 256 rows run in less
+    # once the rest fills three quarters of that time; from four rounds on it
+    # balances by the number of programs. In between, and where an XCD holds a
+    # part of a head, the halves on 4 waves fill the last round better. 256-wide
+    # heads do not fit 256 rows' registers ([64, 2048] 987 / 221)
+    if D <= 128 and S >= 2048 and heads % 8 == 0 and (
+            programs >= 1024 or (376 < programs <= 512 and (heads % 16 == 0 or S > 2304))):
         return 256, 8
     return 128, 4
 

@@ -28,11 +28,14 @@ def test_tile_rule(S, heads, D, causal, want):
 
 
 @pytest.mark.parametrize("S,heads,want", [
-    # heads that the 8 XCDs share evenly, around 352, 512 and 1024 programs
-    (2048, 40, (128, 4)), (4096, 16, (128, 8)), (2816, 32, (128, 4)), (2304, 40, (256, 8)),
-    (2048, 56, (256, 8)), (3072, 40, (256, 8)), (2560, 48, (256, 8)), (4096, 32, (256, 8)),
-    (8192, 16, (256, 8)), (3328, 40, (128, 4)), (2048, 72, (128, 4)), (4096, 56, (128, 4)),
-    (2048, 120, (128, 4)), (4096, 64, (256, 8)), (2048, 136, (256, 8)),
+    # heads that the 8 XCDs share evenly, around 376, 512 and 1024 programs
+    (2048, 40, (128, 4)), (4096, 16, (128, 8)), (2816, 32, (128, 4)), (5888, 16, (128, 4)),
+    (6144, 16, (256, 8)), (3000, 32, (256, 8)), (2560, 40, (256, 8)), (3072, 40, (256, 8)),
+    (2560, 48, (256, 8)), (4096, 32, (256, 8)), (8192, 16, (256, 8)), (3328, 40, (128, 4)),
+    (2048, 72, (128, 4)), (4096, 56, (128, 4)), (2048, 120, (128, 4)), (4096, 64, (256, 8)),
+    (2048, 136, (256, 8)),
+    # an odd number of heads per XCD, 9 blocks and more
+    (2048, 56, (128, 4)), (2304, 56, (128, 4)), (2305, 40, (256, 8)), (4096, 24, (256, 8)),
     # heads that they do not, beside those
     (2048, 47, (128, 4)), (2048, 49, (128, 4)), (2048, 63, (128, 4)), (4096, 31, (128, 4)),
     (2048, 129, (128, 4)), (4096, 65, (128, 4)),
@@ -41,3 +44,8 @@ def test_tile_rule(S, heads, D, causal, want):
 ])
 def test_causal_lines_and_their_neighbours(S, heads, want):
     assert attention_tile(S, heads, 128, True) == want
+
+
+@pytest.mark.parametrize("S,heads", [(2048, 48), (2560, 40), (2048, 128), (4096, 64)])
+def test_wider_heads_keep_four_waves(S, heads):
+    assert attention_tile(S, heads, 256, True) == (128, 4)

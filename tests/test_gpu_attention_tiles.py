@@ -29,3 +29,18 @@ def test_small_launches(B, H, S, D, causal):
             ref = torch.softmax(s, -1) @ v[b, h].double()
             err = (o[b, h].double() - ref).norm(dim=1) / ref.norm(dim=1)
             assert float(err.max()) <= 1e-2, (b, h)
+
+
+@pytest.mark.parametrize("S", [128, 300])
+def test_wide_heads_on_four_waves(S):
+    """256-wide heads on 128 rows, which large causal launches of them take."""
+    from newt_amd import workloads as W
+    g = torch.Generator(device="cuda").manual_seed(S)
+    q, k, v = (torch.randn(1, 2, S, 256, generator=g, device="cuda").bfloat16() for _ in range(3))
+    o = W.attention(q, k, v, causal=True, BLOCK_M=128, num_warps=4)
+    for h in range(2):
+        s = q[0, h].double() @ k[0, h].double().t().contiguous() / 16
+        s.masked_fill_(torch.ones(S, S, dtype=torch.bool, device="cuda").triu(1), float("-inf"))
+        ref = torch.softmax(s, -1) @ v[0, h].double()
+        err = (o[0, h].double() - ref).norm(dim=1) / ref.norm(dim=1)
+        assert float(err.max()) <= 1e-2, h
